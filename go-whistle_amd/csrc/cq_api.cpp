@@ -110,6 +110,10 @@ struct CqStore {
     float cb[16];
     int ncb;
     float cb_max, lut_step, inv_sqrt;
+    // the 4-bit table form's split of the table entries (ResidLevels)
+    bool resid_ok = false;
+    ResidLevels lv{};
+    uint32_t tab_lv[16] = {};  // code c's levels as the bytes of a dword
     uint8_t *d_idx = nullptr;
     uint16_t *d_norm = nullptr;
     size_t idx_bytes = 0, norm_bytes = 0;
@@ -136,6 +140,25 @@ bool uses_lut(const cq_matrix *m) { return !m->exact && m->st->group_bytes <= kL
 float gomax(float a, float b) {
     if (a != a || b != b) return NAN;
     return a > b ? a : b;
+}
+
+// The codebook's levels for the 4-bit table form: finite and with a largest
+// magnitude far from float32's limits, so that cb_max times a scaled value
+// (at most 8191 / cb_max) is exact to a few ulp. Other codebooks take the
+// other forms.
+void fill_resid_levels(CqStore &s) {
+    s.resid_ok = s.width == 4 && s.cb_max >= 0x1p-60f && s.cb_max <= 0x1p60f;  // false for a NaN
+    if (!s.resid_ok) return;
+    for (int c = 0; c < s.ncb; ++c) {
+        const double g = static_cast<double>(s.cb[c]) / s.cb_max;
+        const double c1 = std::nearbyint(127.0 * g), c2 = std::nearbyint(8.0 * g);
+        const double c3 = std::nearbyint(8.0 * (127.0 * g - c1));
+        const double lv[3] = {c1, c2, c3};
+        for (int k = 0; k < 3; ++k) {
+            s.lv.c[k][c] = static_cast<float>(lv[k]);
+            s.tab_lv[c] |= (static_cast<uint32_t>(static_cast<int>(lv[k])) & 255u) << (8 * k);
+        }
+    }
 }
 
 // The shared-table test of lut.go:206-209.
@@ -703,15 +726,16 @@ int run_split(cq_matrix *const *ms, int n, float *const *dsts, const float *x, i
 //
 // A pre-pass builds each activation's tables once and the MFMAs of every
 // 64-row block stream them. A workgroup reads its 32 activations' tables
-// whole (16 KiB per activation and 512 inputs), so the form pays where the
+// whole (8 KiB per activation and 512 inputs), so the form pays where the
 // lut kernel's work, linear in rows x activations, outgrows the form's
 // ~15 us floor at these sizes (from about 256K row-activations at 4 bits,
 // 384K at 2, and 16 activations), or where its (block, tile) workgroups
 // reach the CUs; past 3072 activations over 768 rows or more, at 2 bits,
 // or up to 6144 activations (a 512-row CQ4 matrix's tables, read by few
 // blocks, cost more than the 512-row MFMA form's own table builds at 12000).
-// Measured on MI355X (pre-pass + product against the form chosen
-// otherwise): at 256 activations the four 512x512 CQ4 q/k/v/gate products
+// Measured on MI355X when the lines were drawn (pre-pass + product against
+// the form chosen otherwise; the 4-bit split into planes and residuals has
+// since made the form's times 0.5-0.75 of these, see lut_mfma_tab_kernel): at 256 activations the four 512x512 CQ4 q/k/v/gate products
 // with the norm 18.6 against 28.2 us, 2048x512 CQ2 with the norm and SiLU
 // 16.0 against 19.1 us, the 16384x512 head 60.2 against 64.4 us, 1536x512
 // CQ4 16.2 against 23.5 us, 1024x512 CQ4 15.9 against 16.7 us, but 1024x512
@@ -751,6 +775,7 @@ bool tab_pays(cq_matrix *const *ms, int n, int rows) {
     const CqStore &s0 = *ms[0]->st;
     if (!mfma_geometry_supported(s0.width, s0.group) || s0.groups > std::min(kTabMaxGroups, tab_max_groups()))
         return false;
+    if (s0.width == 4 && !s0.resid_ok) return false;
     long long blocks = 0;
     for (int k = 0; k < n; ++k) {
         if (!uses_lut(ms[k]) || !shares_tables(s0, *ms[k]->st)) return false;
@@ -765,11 +790,11 @@ bool tab_pays(cq_matrix *const *ms, int n, int rows) {
 // whose wavefronts share the tile's A operands through LDS (a quarter of the
 // L2 reads) once such workgroups number two per CU or more; below that the
 // workgroup per block spreads wider. Measured on MI355X (one block, against
-// four): 2048x512 CQ4 at 6000 and 12000 activations 188.4 / 359.7 -> 179.5 /
-// 332.2 us, 2048x1024 CQ4 at 12000 809 -> 615 us, the 16384x512 head at 256,
-// 1500 and 12000 66.8 / 315.7 / 2433 -> 64.5 / 297.3 / 2137 us; 2048x512
-// CQ4 at 1500 (376 slab workgroups) 60.0 -> 66.9 us and at 256 (64) 16.4
-// -> 38.3 us.
+// four): 2048x512 CQ4 at 6000 and 12000 activations 109.7 / 207.6 -> 95.7 /
+// 183.4 us, 2048x1024 CQ4 at 12000 411 -> 356 us, the 16384x512 head at 256,
+// 1500 and 3000 38.3 / 182.1 / 357 -> 35.2 / 160.7 / 313 us; 2048x512 CQ4 at
+// 1500 (376 slab workgroups) 35.8 -> 37.2 us and at 256 (64) 12.4 -> 22.2
+// us.
 int tab_row_blocks(cq_matrix *const *ms, int n, int rows) {
     long long slabs = 0;
     for (int k = 0; k < n; ++k) {
@@ -811,7 +836,9 @@ int run_tab(cq_matrix *const *ms, int n, float *const *dsts, const float *x, int
     for (int c = 0; c < 16; ++c) t.cb[c] = a.jobs[0].cb[c];
     t.cb_max = s0.cb_max;
     t.lut_step = s0.lut_step;
-    const size_t tb = tab_table_bytes(s0.width, s0.groups, tiles), sb = tab_step_bytes(s0.groups, tiles);
+    t.lv = s0.lv;
+    std::memcpy(a.tab_lv, s0.tab_lv, sizeof a.tab_lv);
+    const size_t tb = tab_table_bytes(s0.groups, tiles), sb = tab_step_bytes(s0.groups, tiles);
     WsScope ws;
     char *base = static_cast<char *>(const_cast<void *>(tables));
     if (!base) {
@@ -1085,6 +1112,7 @@ int cq_new(int out, int in, int group, int bits, int width, const float *codeboo
         st->cb[c] = codebook[c];
         st->cb_max = gomax(st->cb_max, std::fabs(codebook[c]));
     }
+    fill_resid_levels(*st);
     st->lut_step = static_cast<float>(1.0 / (kLutQ * std::sqrt(static_cast<double>(group))));  // lut.go:213-215
     st->inv_sqrt = static_cast<float>(1.0 / std::sqrt(static_cast<double>(group)));          // kernel.go:377
 
@@ -1343,7 +1371,7 @@ size_t cq_tables_bytes(int n, cq_matrix *const *ms, int rows) {
     if (!tab_pays(ms, n, rows)) return 0;
     const CqStore &s0 = *ms[0]->st;
     const int tiles = (rows + 31) / 32;
-    return tab_table_bytes(s0.width, s0.groups, tiles) + tab_step_bytes(s0.groups, tiles);
+    return tab_table_bytes(s0.groups, tiles) + tab_step_bytes(s0.groups, tiles);
 }
 
 int cq_gemm_tables_dev(const cq_matrix *m, float *dst, const float *x, const float *gate, int rows, const float *resid,
@@ -1378,7 +1406,7 @@ int cq_gemm_tables_dev(const cq_matrix *m, float *dst, const float *x, const flo
     TabOut to;
     std::memset(&to, 0, sizeof to);
     to.tab = static_cast<int8_t *>(tables);
-    to.stp = reinterpret_cast<float *>(static_cast<char *>(tables) + tab_table_bytes(n0.width, n0.groups, tiles));
+    to.stp = reinterpret_cast<float *>(static_cast<char *>(tables) + tab_table_bytes(n0.groups, tiles));
     to.ngain = next_gain;
     to.in = n0.in;
     to.groups = n0.groups;
@@ -1387,6 +1415,7 @@ int cq_gemm_tables_dev(const cq_matrix *m, float *dst, const float *x, const flo
     for (int c = 0; c < 16; ++c) to.cb[c] = c < n0.ncb ? n0.cb[c] : 0.0f;
     to.cb_max = n0.cb_max;
     to.lut_step = n0.lut_step;
+    to.lv = n0.lv;
     return run_product(&mm, 1, &dst, x, rows, st, &f, &to, built);
 }
 

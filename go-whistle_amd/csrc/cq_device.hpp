@@ -230,6 +230,52 @@ constexpr float kRneMagic = 12582912.0f;  // 1.5 * 2^23
 
 __device__ __forceinline__ uint32_t rne_bits(float f) { return __float_as_uint(f + kRneMagic); }
 
+// One item of the 4-bit table form's tables (ResidLevels, cq_internal.hpp):
+// the positions of scaled rotated values x0 and x1. e6 gets the 32 residuals
+// (x0's 16 codes, then x1's) over 8 as 6-bit floats E2M3, which hold every
+// eighth to +-2 exactly (the convert takes slots 2i from its
+// first operand and 2i + 1 from its second); d the two positions' plane
+// values A1, A2, A3 as the bytes of a dword each. Every operation here is
+// exact but the two roundings to an integer that define v = RNE(cb * x) and
+// A1, and the residual is v - sum_k A_k C_k whatever A1's rounding did.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned int u32x6 __attribute__((ext_vector_type(6)));
+
+template <class Levels>
+__device__ __forceinline__ void resid_item(const float (&cb)[16], const Levels &lv, float cb_max, float x0, float x1,
+                                           u32x6 &e6, uint32_t (&d)[2]) {
+    f32x16 even, odd;
+    const float x[2] = {x0, x1};
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const float al = x[p] * cb_max;  // within +-8191
+        const float a1 = rintf(al * (1.0f / 127.0f));
+        const float a2 = rintf(fmaf(-127.0f, a1, al) * 0.125f);
+        const float a3 = rintf(a1 * 0.125f);
+        d[p] = (static_cast<uint32_t>(static_cast<int>(a1)) & 255u) |
+               (static_cast<uint32_t>(static_cast<int>(a2)) & 255u) << 8 |
+               (static_cast<uint32_t>(static_cast<int>(a3)) & 255u) << 16;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            float e = rintf(cb[c] * x[p]);
+            e = fmaf(-a1, lv.c[0][c], e);
+            e = fmaf(-a2, lv.c[1][c], e);
+            e = fmaf(-a3, lv.c[2][c], e);
+            const int s = 16 * p + c;
+            if (s & 1)
+                odd[s >> 1] = e;
+            else
+                even[s >> 1] = e;
+        }
+    }
+    e6 = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(even, odd, 8.0f);
+}
+
+// A scaled rotated value as the 4-bit tables take it: a value that is not
+// finite (an infinite bound's NaN, an overflowing 8191 / M) gives zero
+// entries, as RNE's low bits do for it in the int8 planes.
+__device__ __forceinline__ float resid_value(float x) { return fabsf(x) <= 3.402823466e+38f ? x : 0.0f; }
+
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // Four entries' bit patterns -> the l plane's 4 bytes (v & 63) and the h

@@ -123,6 +123,24 @@ struct WorkUnit {
 constexpr int kKernargJobs = 8;
 constexpr int kLutWaves = 4;  // wavefronts per workgroup of the lut kernel
 
+// The 4-bit table form's split of a table entry. With x a position's scaled
+// rotated value (|cb x| <= 8191 for every level), the entry is v(c) =
+// RNE(cb[c] x): nearly the product of alpha = cb_max x and gamma_c = cb[c] /
+// cb_max, so most of it is a plain int8 contraction and only a small rest
+// needs the one-hot expansion:
+//
+//   v(c) = A1 C1[c] + A2 C2[c] + A3 C3[c] + e(c)
+//   C1 = RNE(127 gamma), C2 = RNE(8 gamma), C3 = RNE(8 (127 gamma - C1))
+//   A1 = RNE(alpha / 127), A2 = RNE((alpha - 127 A1) / 8), A3 = RNE(A1 / 8)
+//
+// all integers, |A1| <= 65, |A2|, |A3| <= 8. The error of the three products
+// is at most 4 * 1/2 + 8 * 1/2 (the part A1 (127 gamma - C1)) + 4 + 8 * 1/2
+// (the part (alpha - 127 A1) gamma) = 14, and RNE's 1/2: |e| <= 15, exact in
+// the 6-bit float E2M3, whose MFMA runs at twice int8's rate.
+struct ResidLevels {
+    float c[3][16];
+};
+
 // The next product's tables, built in a producer's epilogue (the table
 // form's pre-pass, fused): when a workgroup holds all of its activation's
 // output row y, it writes the tables and steps of ZCRMSNorm(y; ngain)
@@ -136,6 +154,7 @@ struct TabOut {
     int in, groups, bits, tiles;
     float cb[16];
     float cb_max, lut_step;
+    ResidLevels lv;  // 4 bits
 };
 
 struct LutLaunch {
@@ -164,6 +183,7 @@ struct LutLaunch {
     const int8_t *tab;
     const float *tstp;
     int tab_at, tab_nb;
+    uint32_t tab_lv[16];  // 4 bits: code c's plane levels C1, C2, C3 as the bytes of a dword
     int tab_rb;  // row blocks per workgroup of the product: 1, or 4 sharing the A operands (tab_nb, wg0 count slabs)
     // The lut kernel's wide form, one workgroup per activation over all of
     // one job's rows: the next product's tables (tout.tab null: none).
@@ -176,6 +196,11 @@ struct LutLaunch {
 // [tile][group][position pair][plane][half][32][16 codes] (a wavefront's
 // MFMA A operand of one plane and pair is 1 KiB contiguous), and the
 // groups' steps [tile][group][32]. Activations past rows get zero tables.
+// 2 bits: both int8 planes, as above. 4 bits: the split of ResidLevels,
+// [tile][group][8 positions (16)]: lane 32 h + act holds positions 4q + 2h and
+// 4q + 2h + 1 of the two 64-wide MFMA steps q, its residuals (2 steps of 24
+// bytes) as three 16-byte pieces [3][64][16], then the planes [64][4 positions]
+// [A1, A2, A3, 0].
 struct TabArgs {
     const float *x;
     long long x_stride;
@@ -184,11 +209,14 @@ struct TabArgs {
     int rows, in, groups, tiles;
     float cb[16];
     float cb_max, lut_step;
+    ResidLevels lv;  // 4 bits
     int8_t *tab;
     float *stp;
 };
+constexpr int kTabGroupBytes = 65536;  // a tile's tables of one group, at either width
+constexpr int kTabUnitBytes = 4096;    // 4 bits: the tables of 8 positions
 // Bytes of the tables and of the steps for `tiles` tiles of 32 activations.
-size_t tab_table_bytes(int bits, int groups, int tiles);
+size_t tab_table_bytes(int groups, int tiles);
 size_t tab_step_bytes(int groups, int tiles);
 // Groups the product kernel's LDS holds terms for.
 int tab_max_groups();

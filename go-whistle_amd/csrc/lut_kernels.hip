@@ -448,13 +448,36 @@ __device__ __forceinline__ void next_tables(const TabOut &o, const float *yo, un
         const float m = o.cb_max * mx;
         const float inv = m > 0.0f ? static_cast<float>(kLutQ) / m : 0.0f;  // lutInv (lut.go:219-225)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) av[g * AP + e * 64 + lane] = v[e] * inv;
+        for (int e = 0; e < 2; ++e) {
+            const float sv = v[e] * inv;
+            av[g * AP + e * 64 + lane] = TB == 4 ? resid_value(sv) : sv;
+        }
         if (lane == 0) stp[(static_cast<size_t>(t >> 5) * groups + g) * 32 + (t & 31)] = m * o.lut_step;
     }
     __syncthreads();
     float cbv[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) cbv[q] = o.cb[q];
+    if constexpr (TB == 4) {  // an item is two positions of one lane half (tab4_item, mfma_kernels.hip)
+        CQ_GLOBAL int8_t *base = gptr_w(o.tab) + static_cast<size_t>(t >> 5) * groups * kTabGroupBytes;
+        for (int it = tid; it < groups * 64; it += 64 * W) {
+            const int g = it >> 6, q = (it >> 1) & 31, h = it & 1, ln = h * 32 + (t & 31);
+            const float *x = av + g * AP + 4 * q + 2 * h;
+            u32x6 e;
+            uint32_t d[2];
+            resid_item(cbv, o.lv, o.cb_max, x[0], x[1], e, d);
+            CQ_GLOBAL int8_t *u = base + static_cast<size_t>(g) * kTabGroupBytes + (q >> 1) * kTabUnitBytes + ln * 16;
+            if (q & 1) {
+                *reinterpret_cast<CQ_GLOBAL uint2 *>(u + 1024 + 8) = make_uint2(e[0], e[1]);
+                *reinterpret_cast<CQ_GLOBAL uint4 *>(u + 2048) = make_uint4(e[2], e[3], e[4], e[5]);
+            } else {
+                *reinterpret_cast<CQ_GLOBAL uint4 *>(u) = make_uint4(e[0], e[1], e[2], e[3]);
+                *reinterpret_cast<CQ_GLOBAL uint2 *>(u + 1024) = make_uint2(e[4], e[5]);
+            }
+            *reinterpret_cast<CQ_GLOBAL uint2 *>(u + 3072 + (q & 1) * 8) = make_uint2(d[0], d[1]);
+        }
+        return;
+    }
     CQ_GLOBAL int8_t *tab = gptr_w(o.tab) + (static_cast<size_t>(t >> 5) * groups) * NP * 2048 + (t & 31) * 16;
     for (int it = tid; it < groups * NJ; it += 64 * W) {
         const int g = it / NJ, j = it - g * NJ;

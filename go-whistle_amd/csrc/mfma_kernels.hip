@@ -50,6 +50,8 @@ namespace {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x8 __attribute__((ext_vector_type(8)));
 
 template <int BITS>
 struct MfmaGeo {
@@ -1027,15 +1029,129 @@ hipError_t launch_split_t(const LutLaunch &a, int grid, hipStream_t s) {
 // lut kernel looks every entry up once per activation. The table form
 // builds each activation's tables once: lut_tables_kernel rotates and
 // bounds each (activation, group) and writes the int8 planes of its 16-entry
-// tables, in the A-operand order of v_mfma_i32_32x32x32_i8, and the group's
-// step; lut_mfma_tab_kernel streams them into the MFMAs of every row tile,
+// tables (4 bits: the split of ResidLevels), in the MFMAs' A-operand order,
+// and the group's step; lut_mfma_tab_kernel streams them into the MFMAs of every row tile,
 // 64 rows x 32 activations a workgroup, its four wavefronts taking the
 // groups in turn. The arithmetic is the split form's, so the result is bit
 // for bit the lut kernel's.
 constexpr int kTabWaves = 4;      // wavefronts per workgroup of the product
 constexpr int kTabDepth = 4;      // position pairs of A operands in flight per wavefront
+constexpr int kTabDepth4 = 3;     // 4 bits: units of 8 positions of A operands in flight per wavefront
 constexpr int kTabMaxGroups = 16;  // groups whose terms the product's LDS holds
 constexpr int kTabPre4Rows = 3072;  // activations up to which the pre-pass takes 4 a workgroup
+
+// 4 bits: a wavefront's share of the tables of 8 positions (a unit), lane
+// (half h, activation): the residuals of the unit's two 64-wide steps, 6
+// dwords each in three 16-byte reads, and the planes of the lane's four
+// positions (TabArgs' layout).
+struct TabUnit {
+    i32x4 e[3];
+    i32x4 pl;
+};
+template <class P>
+__device__ __forceinline__ TabUnit tab_unit(const P *u, int lane) {
+    TabUnit r;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) r.e[k] = *reinterpret_cast<const i32x4 *>(u + k * 1024 + lane * 16);
+    r.pl = *reinterpret_cast<const i32x4 *>(u + 3072 + lane * 16);
+    return r;
+}
+
+// The same unit's weight operand for one row. A one-hot of 16 4-bit floats
+// (1.0 is 2) is a 64-bit shift by 4 * code; the planes' levels of a code come
+// from a table in LDS (a dword a code, so 4 * code is its offset too).
+struct TabHot {
+    uint32_t o[4];  // 4 * code of the lane's four positions
+    i32x4 hot[2];   // the two steps' one-hots
+    i32x4 lv;       // the positions' levels
+};
+// w holds the row's four nibbles of the lane's half in bytes 0 and 2.
+__device__ __forceinline__ void tab_codes(TabHot &b, uint32_t w) {
+    const uint32_t lo = w << 2, hi = w >> 2;
+    b.o[0] = and_byte<0>(0x3cu, lo);
+    b.o[1] = and_byte<0>(0x3cu, hi);
+    b.o[2] = and_byte<2>(0x3cu, lo);
+    b.o[3] = and_byte<2>(0x3cu, hi);
+}
+__device__ __forceinline__ void tab_levels(TabHot &b, const uint32_t *lv) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        b.lv[k] = *reinterpret_cast<const int *>(reinterpret_cast<const char *>(lv) + b.o[k]);
+}
+__device__ __forceinline__ void tab_hots(TabHot &b) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const unsigned long long h = 2ull << b.o[k];
+        b.hot[k >> 1][2 * (k & 1)] = static_cast<int>(h);
+        b.hot[k >> 1][2 * (k & 1) + 1] = static_cast<int>(h >> 32);
+    }
+}
+// Step s of a unit: 32 activations x 32 rows, 4 positions. The operand's
+// values are e / 8, so the sums are multiples of 1/8 far below 2^21, which
+// float32 adds exactly; 8 times them and the planes' int32 sums make the
+// group's integer (below 2^21), also exactly.
+__device__ __forceinline__ f32x16 tab_mma(const TabUnit &u, const TabHot &b, int s, f32x16 acc) {
+    i32x8 A;
+    if (s == 0)
+        A = i32x8{u.e[0].x, u.e[0].y, u.e[0].z, u.e[0].w, u.e[1].x, u.e[1].y, 0, 0};
+    else
+        A = i32x8{u.e[1].z, u.e[1].w, u.e[2].x, u.e[2].y, u.e[2].z, u.e[2].w, 0, 0};
+    const i32x8 B = {b.hot[s].x, b.hot[s].y, b.hot[s].z, b.hot[s].w, 0, 0, 0, 0};
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B, acc, 2, 4, 0, 0, 0, 0);  // E2M3 times E2M1
+}
+// One unit of a wavefront's 64 rows x 32 activations: 6 MFMAs (two steps of
+// residuals and the planes, on two row tiles), the next unit's reads and
+// operands issued between them in three blocks, so that every LDS read has
+// at least a unit's MFMAs to land in and the VALU runs under the MFMAs (left
+// to itself the compiler put all six behind the VALU, or the planes' first).
+// next_a() reads the next unit into An; w0, w1 are the next unit's index
+// words of the two row tiles.
+template <bool NEXT, class F>
+__device__ __forceinline__ void tab_unit_step(const TabUnit &A, const TabHot (&B)[2], f32x16 (&ae)[2], i32x16 (&ad)[2],
+                                              TabHot (&Bn)[2], uint32_t w0, uint32_t w1, const uint32_t *lv, F next_a) {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) ae[rt] = tab_mma(A, B[rt], 0, ae[rt]);
+    if constexpr (NEXT) {
+        next_a();
+        tab_codes(Bn[0], w0);
+        tab_codes(Bn[1], w1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) ae[rt] = tab_mma(A, B[rt], 1, ae[rt]);
+    if constexpr (NEXT) {
+        tab_levels(Bn[0], lv);
+        tab_hots(Bn[0]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) ad[rt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A.pl, B[rt].lv, ad[rt], 0, 0, 0);
+    if constexpr (NEXT) {
+        tab_levels(Bn[1], lv);
+        tab_hots(Bn[1]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Items of an activation's 4-bit tables of one group (x: the group's scaled
+// rotated values; base: the tile's tables of the group). Item it: step q = it
+// / 2, half h = it % 2, the positions 4q + 2h and 4q + 2h + 1.
+__device__ __forceinline__ void tab4_item(int8_t *base, int it, int act, const float (&cb)[16], const ResidLevels &lv,
+                                          float cb_max, const float *x) {
+    const int q = it >> 1, h = it & 1;
+    u32x6 e;
+    uint32_t d[2];
+    resid_item(cb, lv, cb_max, x[4 * q + 2 * h], x[4 * q + 2 * h + 1], e, d);
+    int8_t *u = base + (q >> 1) * kTabUnitBytes + (h * 32 + act) * 16;
+    if (q & 1) {
+        *reinterpret_cast<uint2 *>(u + 1024 + 8) = make_uint2(e[0], e[1]);
+        *reinterpret_cast<uint4 *>(u + 2048) = make_uint4(e[2], e[3], e[4], e[5]);
+    } else {
+        *reinterpret_cast<uint4 *>(u) = make_uint4(e[0], e[1], e[2], e[3]);
+        *reinterpret_cast<uint2 *>(u + 1024) = make_uint2(e[4], e[5]);
+    }
+    *reinterpret_cast<uint2 *>(u + 3072 + (q & 1) * 8) = make_uint2(d[0], d[1]);
+}
 
 // The pre-pass: a workgroup per TT activations (4 or 8) and one group g.
 // Wavefront w rotates activations w, w + 4, ... (two values per lane), then
@@ -1200,7 +1316,10 @@ __global__ __launch_bounds__(256) void lut_tables_kernel(TabArgs a) {
             const float m = a.cb_max * mx[k];
             const float inv = m > 0.0f ? static_cast<float>(kLutQ) / m : 0.0f;  // lutInv (lut.go:219-225)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) av[tt * AP + e * 64 + lane] = v[k][e] * inv;
+            for (int e = 0; e < 2; ++e) {
+                const float sv = v[k][e] * inv;
+                av[tt * AP + e * 64 + lane] = BITS == 4 ? resid_value(sv) : sv;
+            }
             if (lane == 0) a.stp[(static_cast<size_t>(t >> 5) * a.groups + g) * 32 + (t & 31)] = m * a.lut_step;
         }
     }
@@ -1211,6 +1330,12 @@ __global__ __launch_bounds__(256) void lut_tables_kernel(TabArgs a) {
 #pragma unroll
     for (int q = 0; q < 16; ++q) cbv[q] = a.cb[q];
     const int tt = tid % TT, jb = tid / TT, t = t0 + tt;
+    if constexpr (BITS == 4) {
+        int8_t *base = a.tab + (static_cast<size_t>(t >> 5) * a.groups + g) * kTabGroupBytes;
+#pragma unroll 1
+        for (int it = jb; it < 64; it += PS) tab4_item(base, it, t & 31, cbv, a.lv, a.cb_max, av + tt * AP);
+        return;
+    }
     int8_t *base = a.tab + (static_cast<size_t>(t >> 5) * a.groups + g) * NP * 2048 + (t & 31) * 16;
 #pragma unroll
     for (int k = 0; k < NJ / PS; ++k) {
@@ -1245,6 +1370,19 @@ __global__ __launch_bounds__(256) void lut_tables_kernel(TabArgs a) {
     }
 }
 
+// The 4-bit tables. The one-hot form needs 16 codes a position, and an entry
+// of 14 bits two int8 planes of them: 256 MFMAs of 32 cycles per group for 64
+// rows x 32 activations, as much LDS traffic as MFMA time. With the entries
+// split (ResidLevels) a group takes 64 MFMAs on residuals of 6-bit floats
+// (4 positions each, at twice int8's rate: 8.55 POP/s measured against 4.2)
+// and 32 int8 MFMAs on the planes, 4 bytes a position, and the tables are
+// half the bytes. Measured on MI355X (pre-pass + product, int8 planes, then
+// split): 2048x512 CQ4 at 12,000 activations 309 -> 178 us, at 1,500 53.4 ->
+// 36 us, at 256 16.4 -> 12.4 us; the 16384x512 head at 256 64.5 -> 35 us; the
+// batch-256 decode step 1.525 -> 1.443 ms. What bounds the large ones now is
+// issue: the MFMAs are busy 48% of the cycles, VALU takes as many (the
+// one-hots' shifts and masks, the fold's 5 operations a sum).
+//
 // The product: a workgroup per (64-row block, 32-activation tile), a
 // tile's workgroups on one XCD (or two), which shares their tables in its L2.
 // Wavefront w takes groups w, w + 4, ...: per position pair it reads the
@@ -1279,8 +1417,11 @@ __global__ __launch_bounds__(64 * kTabWaves) void lut_mfma_tab_kernel(LutLaunch 
     const int blk = rb - a.wg0[jb];
     if (blk >= J.nblk) return;  // the whole workgroup
     const int groups = J.groups, units = J.units;
-    int8_t *ohot = reinterpret_cast<int8_t *>(terms + groups * 32 * TP);  // [16][16]: entry c is the one-hot of c
-    if (tid < 16) {
+    int8_t *ohot = reinterpret_cast<int8_t *>(terms + groups * 32 * TP);  // 2 bits: [16][16], entry c the one-hot of c
+    __shared__ uint32_t lvt[16];  // 4 bits: entry c the plane levels of c (static: an address known to the compiler)
+    if (BITS == 4) {
+        if (tid < 16) lvt[tid] = a.tab_lv[tid];
+    } else if (tid < 16) {
         const uint32_t one = 1u << (8 * (tid & 3)), d = tid >> 2;
         *reinterpret_cast<uint4 *>(ohot + tid * 16) =
             make_uint4(d == 0 ? one : 0u, d == 1 ? one : 0u, d == 2 ? one : 0u, d == 3 ? one : 0u);
@@ -1307,12 +1448,18 @@ __global__ __launch_bounds__(64 * kTabWaves) void lut_mfma_tab_kernel(LutLaunch 
     }
 
     for (int g = w; g < groups; g += kTabWaves) {
-        const int8_t *A = a.tab + (static_cast<size_t>(at) * groups + g) * NP * 2048 + lane * 16;
+        const int8_t *A = a.tab + (static_cast<size_t>(at) * groups + g) * kTabGroupBytes + (BITS == 4 ? 0 : lane * 16);
         i32x4 Al[D], Ah[D];
+        TabUnit AU[kTabDepth4];
+        if constexpr (BITS == 4) {
 #pragma unroll
-        for (int p = 0; p < D; ++p) {
-            Al[p] = *reinterpret_cast<const i32x4 *>(A + p * 2048);
-            Ah[p] = *reinterpret_cast<const i32x4 *>(A + p * 2048 + 1024);
+            for (int m = 0; m < kTabDepth4; ++m) AU[m] = tab_unit(A + m * kTabUnitBytes, lane);
+        } else {
+#pragma unroll
+            for (int p = 0; p < D; ++p) {
+                Al[p] = *reinterpret_cast<const i32x4 *>(A + p * 2048);
+                Ah[p] = *reinterpret_cast<const i32x4 *>(A + p * 2048 + 1024);
+            }
         }
         uint32_t idx[M::UPG][2][4];
 #pragma unroll
@@ -1337,51 +1484,90 @@ __global__ __launch_bounds__(64 * kTabWaves) void lut_mfma_tab_kernel(LutLaunch 
             lds_barrier();  // the one-hot table is whole
             first = false;
         }
-        // this half's nibble of pair k in the high nibble of byte k: a
-        // one-hot's offset in the table is one SDWA and
+        float sums[2][16];  // the group's exact integer sums
+        if constexpr (BITS == 4) {
 #pragma unroll
-        for (int u = 0; u < M::UPG; ++u)
+            for (int u = 0; u < M::UPG; ++u)
 #pragma unroll
-            for (int rt = 0; rt < 2; ++rt)
+                for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) idx[u][rt][e] = (idx[u][rt][e] >> hs) << 4;
-        auto onehot = [&](int rt, int pp) -> i32x4 {
-            const uint32_t w4 = idx[pp >> 4][rt][(pp >> 2) & 3];
-            uint32_t off;
-            switch (pp & 3) {
-                case 0: off = and_byte<0>(0xf0u, w4); break;
-                case 1: off = and_byte<1>(0xf0u, w4); break;
-                case 2: off = and_byte<2>(0xf0u, w4); break;
-                default: off = and_byte<3>(0xf0u, w4); break;
-            }
-            return *reinterpret_cast<const i32x4 *>(ohot + off);
-        };
-        i32x4 B[2][2];
+                    for (int e = 0; e < 4; ++e) idx[u][rt][e] = idx[u][rt][e] >> (2 * hs);
+            f32x16 ae[2] = {f32x16{}, f32x16{}};
+            i32x16 ad[2] = {i32x16{}, i32x16{}};
+            auto word = [&](int rt, int m) { return idx[m >> 2][rt][m & 3]; };
+            TabHot B[2][2];
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) B[0][rt] = onehot(rt, 0);
-        i32x16 accl[2] = {i32x16{}, i32x16{}}, acch[2] = {i32x16{}, i32x16{}};
-#pragma unroll
-        for (int pp = 0; pp < NP; ++pp) {
-            const int s = pp % D, sb = pp & 1;
-            if (pp + 1 < NP) {
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt) B[sb ^ 1][rt] = onehot(rt, pp + 1);
-            }
-            __builtin_amdgcn_sched_barrier(0);  // the next pair's one-hot reads go out before these MFMAs
-#pragma unroll
-            for (int rt = 0; rt < 2; ++rt)
-                accl[rt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(Al[s], B[sb][rt], accl[rt], 0, 0, 0);
-#pragma unroll
-            for (int rt = 0; rt < 2; ++rt)
-                acch[rt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(Ah[s], B[sb][rt], acch[rt], 0, 0, 0);
-            // the slot's next pair goes out here, kTabDepth pairs before its
-            // use (the compiler would otherwise move the loads next to it)
-            __builtin_amdgcn_sched_barrier(0);
-            if (pp + D < NP) {
-                Al[s] = *reinterpret_cast<const i32x4 *>(A + (pp + D) * 2048);
-                Ah[s] = *reinterpret_cast<const i32x4 *>(A + (pp + D) * 2048 + 1024);
+            for (int rt = 0; rt < 2; ++rt) {
+                tab_codes(B[0][rt], word(rt, 0));
+                tab_levels(B[0][rt], lvt);
+                tab_hots(B[0][rt]);
             }
             __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < 16; ++m) {
+                const int sl = m % kTabDepth4, sb = m & 1;
+                if (m + 1 < 16)
+                    tab_unit_step<true>(AU[sl], B[sb], ae, ad, B[sb ^ 1], word(0, m + 1), word(1, m + 1), lvt, [] {});
+                else
+                    tab_unit_step<false>(AU[sl], B[sb], ae, ad, B[sb ^ 1], 0, 0, lvt, [] {});
+                if (m + kTabDepth4 < 16) AU[sl] = tab_unit(A + (m + kTabDepth4) * kTabUnitBytes, lane);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sums[rt][i] = fmaf(8.0f, ae[rt][i], static_cast<float>(ad[rt][i]));
+        } else {
+            // this half's nibble of pair k in the high nibble of byte k: a
+            // one-hot's offset in the table is one SDWA and
+#pragma unroll
+            for (int u = 0; u < M::UPG; ++u)
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) idx[u][rt][e] = (idx[u][rt][e] >> hs) << 4;
+            auto onehot = [&](int rt, int pp) -> i32x4 {
+                const uint32_t w4 = idx[pp >> 4][rt][(pp >> 2) & 3];
+                uint32_t off;
+                switch (pp & 3) {
+                    case 0: off = and_byte<0>(0xf0u, w4); break;
+                    case 1: off = and_byte<1>(0xf0u, w4); break;
+                    case 2: off = and_byte<2>(0xf0u, w4); break;
+                    default: off = and_byte<3>(0xf0u, w4); break;
+                }
+                return *reinterpret_cast<const i32x4 *>(ohot + off);
+            };
+            i32x4 B[2][2];
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt) B[0][rt] = onehot(rt, 0);
+            i32x16 accl[2] = {i32x16{}, i32x16{}}, acch[2] = {i32x16{}, i32x16{}};
+#pragma unroll
+            for (int pp = 0; pp < NP; ++pp) {
+                const int s = pp % D, sb = pp & 1;
+                if (pp + 1 < NP) {
+#pragma unroll
+                    for (int rt = 0; rt < 2; ++rt) B[sb ^ 1][rt] = onehot(rt, pp + 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // the next pair's one-hot reads go out before these MFMAs
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt)
+                    accl[rt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(Al[s], B[sb][rt], accl[rt], 0, 0, 0);
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt)
+                    acch[rt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(Ah[s], B[sb][rt], acch[rt], 0, 0, 0);
+                // the slot's next pair goes out here, kTabDepth pairs before its
+                // use (the compiler would otherwise move the loads next to it)
+                __builtin_amdgcn_sched_barrier(0);
+                if (pp + D < NP) {
+                    Al[s] = *reinterpret_cast<const i32x4 *>(A + (pp + D) * 2048);
+                    Ah[s] = *reinterpret_cast<const i32x4 *>(A + (pp + D) * 2048 + 1024);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sums[rt][i] = static_cast<float>(accl[rt][i] + 64 * acch[rt][i]);
         }
         float nrm[2];
 #pragma unroll
@@ -1391,9 +1577,8 @@ __global__ __launch_bounds__(64 * kTabWaves) void lut_mfma_tab_kernel(LutLaunch 
             const int tt = (i >> 2) * 8 + half * 4 + (i & 3);
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
-                const int sum = accl[rt][i] + 64 * acch[rt][i];
                 const float coef = nrm[rt] * st[i];
-                terms[(g * 32 + tt) * TP + rt * 32 + l32] = static_cast<float>(sum) * coef;
+                terms[(g * 32 + tt) * TP + rt * 32 + l32] = sums[rt][i] * coef;
             }
         }
     }
@@ -1435,7 +1620,10 @@ __global__ __launch_bounds__(64 * kTabWaves) void lut_mfma_tab_kernel(LutLaunch 
 // load the compiler tracks is in flight in the loop (it would wait for the
 // DMAs behind it). Each wavefront folds its rows' terms in registers in
 // group order from 0 (lut.go:297-310), then runs the lut kernel's epilogue
-// on its block.
+// on its block: from the accumulators as they lie (12,000 activations 203 ->
+// 178 us: the walk through LDS and the general epilogue cost as much as one
+// group's MFMAs), through LDS only for the K/V append, which needs lane =
+// row.
 constexpr int kSaPairs = 8;   // position pairs per ring slot (16 KiB)
 constexpr int kSaSlots = 3;   // ring slots: kSaSlots - 1 in flight while one is read
 constexpr int kSaAhead = kSaSlots - 1;
@@ -1478,17 +1666,18 @@ constexpr size_t sa_lds_bytes() {
 template <int BITS>
 __global__ __launch_bounds__(64 * kSaBlocks, 2) void lut_mfma_tabs_kernel(LutLaunch a) {
     using M = MfmaGeo<BITS>;
-    constexpr int NP = M::NJ / 2, SPG = NP / kSaPairs, UPG = M::UPG, AUX = UPG + 2;
+    constexpr int SPG = kTabGroupBytes / kSaSlot, UPG = M::UPG, AUX = UPG + 2;
     // a group's aux loads go out at its second step and must be older than
     // the next group's first slot
-    static_assert(NP % kSaPairs == 0 && SPG >= kSaAhead + 2, "a group's steps");
+    static_assert(SPG >= kSaAhead + 2, "a group's steps");
+    static_assert(BITS == 4 || (M::NJ / 2) * 2048 == kTabGroupBytes, "a group's tables");
     static_assert(kSaDma * (kSaAhead - 1) + AUX <= 15, "the wait counts fit sa_wait_vm");
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned char *ring = smem;                                            // [slot][pair][plane][64][16]
     unsigned char *idxl = ring + kSaSlots * kSaSlot;                       // [wave][unit][64 rows][16]
     unsigned char *nrml = idxl + kSaBlocks * UPG * 1024;                   // [wave][64 fp16 norms]
     unsigned char *stpl = nrml + kSaBlocks * 128;                          // [wave][32 steps]
-    int8_t *ohot = reinterpret_cast<int8_t *>(stpl + kSaBlocks * 128);     // [16][16]: entry c is the one-hot of c
+    int8_t *ohot = reinterpret_cast<int8_t *>(stpl + kSaBlocks * 128);     // as lut_mfma_tab_kernel's
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, half = lane >> 5, l32 = lane & 31;
     const int nat = a.tab_at, L = blockIdx.x;
     // workgroup L on XCD L % 8 as its (L / 8)-th; the (tile, slab) items,
@@ -1509,12 +1698,15 @@ __global__ __launch_bounds__(64 * kSaBlocks, 2) void lut_mfma_tabs_kernel(LutLau
     const int blk = blkS + (mine ? w : nbh - 1);
     const size_t bk = static_cast<size_t>(J.blk0 + blk);
     const int groups = J.groups, units = J.units, nsteps = groups * SPG;
-    if (tid < 16) {
+    __shared__ uint32_t lvt[16];
+    if (BITS == 4) {
+        if (tid < 16) lvt[tid] = a.tab_lv[tid];
+    } else if (tid < 16) {
         const uint32_t one = 1u << (8 * (tid & 3)), d = tid >> 2;
         *reinterpret_cast<uint4 *>(ohot + tid * 16) =
             make_uint4(d == 0 ? one : 0u, d == 1 ? one : 0u, d == 2 ? one : 0u, d == 3 ? one : 0u);
     }
-    const int8_t *T = a.tab + static_cast<size_t>(at) * groups * NP * 2048;  // the tile's A operands
+    const int8_t *T = a.tab + static_cast<size_t>(at) * groups * kTabGroupBytes;  // the tile's A operands
     const uint8_t *IDX = J.idx;
     // the ring's step k: kSaSlot bytes of T into slot k % kSaSlots, 1 KiB a wavefront load
     auto dma_step = [&](int k) {
@@ -1547,7 +1739,8 @@ __global__ __launch_bounds__(64 * kSaBlocks, 2) void lut_mfma_tabs_kernel(LutLau
         uint32_t idx[UPG][2][4];
         unsigned short nrm16[2];
         float st[16];
-        i32x16 accl[2] = {i32x16{}, i32x16{}}, acch[2] = {i32x16{}, i32x16{}};
+        i32x16 accl[2] = {i32x16{}, i32x16{}}, acch[2] = {i32x16{}, i32x16{}};  // 4 bits: accl the planes'
+        f32x16 ae[2] = {f32x16{}, f32x16{}};                                   // 4 bits: the residuals' sums
         const bool aux_next = g + 1 < groups;
 #pragma unroll
         for (int s = 0; s < SPG; ++s) {
@@ -1566,10 +1759,10 @@ __global__ __launch_bounds__(64 * kSaBlocks, 2) void lut_mfma_tabs_kernel(LutLau
 #pragma unroll
                     for (int rt = 0; rt < 2; ++rt) {
                         const uint4 v = *reinterpret_cast<const uint4 *>(idxl + (w * UPG + u) * 1024 + (rt * 32 + l32) * 16);
-                        idx[u][rt][0] = (v.x >> hs) << 4;
-                        idx[u][rt][1] = (v.y >> hs) << 4;
-                        idx[u][rt][2] = (v.z >> hs) << 4;
-                        idx[u][rt][3] = (v.w >> hs) << 4;
+                        const uint32_t vw[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            idx[u][rt][e] = BITS == 4 ? vw[e] >> (2 * hs) : (vw[e] >> hs) << 4;
                     }
 #pragma unroll
                 for (int rt = 0; rt < 2; ++rt)
@@ -1579,6 +1772,31 @@ __global__ __launch_bounds__(64 * kSaBlocks, 2) void lut_mfma_tabs_kernel(LutLau
                 for (int i = 0; i < 16; ++i) st[i] = sp[(i >> 2) * 8 + (i & 3)];
             }
             if (s == 1 && aux_next) dma_aux(g + 1);  // the buffers were read out at s = 0 (barrier between)
+            if constexpr (BITS == 4) {
+                constexpr int UPS = kSaSlot / kTabUnitBytes;  // units of 8 positions in a slot
+                const unsigned char *sl = ring + (k % kSaSlots) * kSaSlot;
+                auto word = [&](int rt, int m) { return idx[m >> 2][rt][m & 3]; };
+                TabUnit A[2];
+                TabHot B[2][2];
+                A[0] = tab_unit(sl, lane);
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt) {
+                    tab_codes(B[0][rt], word(rt, s * UPS));
+                    tab_levels(B[0][rt], lvt);
+                    tab_hots(B[0][rt]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int p = 0; p < UPS; ++p) {
+                    const int c = p & 1, m = s * UPS + p + 1;
+                    if (p + 1 < UPS)
+                        tab_unit_step<true>(A[c], B[c], ae, accl, B[c ^ 1], word(0, m), word(1, m), lvt,
+                                            [&] { A[c ^ 1] = tab_unit(sl + (p + 1) * kTabUnitBytes, lane); });
+                    else
+                        tab_unit_step<false>(A[c], B[c], ae, accl, B[c ^ 1], 0, 0, lvt, [] {});
+                }
+                continue;
+            }
             // this half's nibble of pair pp in the high nibble of byte pp: a
             // one-hot's offset in the table is one SDWA and
             auto onehot = [&](int rt, int pp) -> i32x4 {
@@ -1625,13 +1843,50 @@ __global__ __launch_bounds__(64 * kSaBlocks, 2) void lut_mfma_tabs_kernel(LutLau
         for (int i = 0; i < 16; ++i)
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
-                const int sum = accl[rt][i] + 64 * acch[rt][i];
+                const float sum = BITS == 4 ? fmaf(8.0f, ae[rt][i], static_cast<float>(accl[rt][i]))
+                                            : static_cast<float>(accl[rt][i] + 64 * acch[rt][i]);
                 const float coef = nrm[rt] * st[i];
-                const float t = static_cast<float>(sum) * coef;
+                const float t = sum * coef;
                 y[rt][i] = y[rt][i] + t;
             }
     }
-    // y to lane = row through LDS (the ring, read out by every wavefront)
+    if (!J.app_q) {
+        // y straight from the accumulators: register i of a lane is activation
+        // (i / 4) * 8 + half * 4 + i % 4 and row l32 of a row tile, so 32
+        // lanes write 128 contiguous bytes of one activation's row.
+        if (!mine) return;
+        const int t0 = at * 32 + half * 4, r0 = (J.blk0 + blk) * 64 + l32 - J.row0;  // view row of tile 0
+        const long long ys = J.y_stride, rs = J.resid_stride;
+        const int rows = J.rows, out = J.out, act = J.act;
+        const float *R = J.resid;
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+            const int r = r0 + rt * 32;
+            if (r < 0 || r >= out) continue;
+            float *Y = J.y + t0 * ys + r;
+            if (R) {
+                const float *Q = R + t0 * rs + r;
+                float rv[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int tt = (i >> 2) * 8 + (i & 3);
+                    rv[i] = t0 + tt < rows ? Q[tt * rs] : 0.0f;
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) y[rt][i] = rv[i] + y[rt][i];
+            } else if (act == 1) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) y[rt][i] = silu_value(y[rt][i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int tt = (i >> 2) * 8 + (i & 3);
+                if (t0 + tt < rows) Y[tt * ys] = y[rt][i];
+            }
+        }
+        return;
+    }
+    // the append: y to lane = row through LDS (the ring, read out by every wavefront)
     __builtin_amdgcn_s_waitcnt(0);
     lds_barrier();
     float *tr = reinterpret_cast<float *>(ring) + w * 32 * 64;  // [activation][row]
@@ -1716,10 +1971,7 @@ hipError_t launch_lut_mfma_split(const LutLaunch &a, int bits, int fold_blocks, 
     return hipGetLastError();
 }
 
-size_t tab_table_bytes(int bits, int groups, int tiles) {
-    const int np = bits == 4 ? MfmaGeo<4>::NJ / 2 : MfmaGeo<2>::NJ / 2;
-    return static_cast<size_t>(tiles) * groups * np * 2048;
-}
+size_t tab_table_bytes(int groups, int tiles) { return static_cast<size_t>(tiles) * groups * kTabGroupBytes; }
 
 size_t tab_step_bytes(int groups, int tiles) { return static_cast<size_t>(tiles) * groups * 32 * sizeof(float); }
 

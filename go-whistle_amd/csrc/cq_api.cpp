@@ -960,10 +960,56 @@ int run_dense(cq_matrix *const *ms, int n, float *const *dsts, const float *x, i
     return ws_release(ws.l);
 }
 
+// ---- few rows ----
+
+// Products of few rows over all their matrices, which share their tables:
+// evaluated without tables (lut_few_kernel). A workgroup is one activation,
+// kFewWaves wavefronts at most of one group and 32 rows each. Its time grows
+// with rows x activations where the forms with tables pay the tables once an
+// activation, so past one set of 32 rows it runs to kFewWork sets x
+// activations. Measured on MI355X (us, few against the form chosen
+// otherwise): 96x512 CQ4 at 1, 375, 1500 and 3000 activations 5.2, 6.7, 14.4,
+// 25.0 against 5.7, 8.0, 20.8, 23.9; 128x512 CQ2 at 1, 750 and 1500 4.6, 8.2,
+// 13.3 against 5.2, 9.5, 11.2; 512x128 CQ4 at 375 and 1500 7.4, 17.1 against
+// 10.2, 12.3; one set of rows wins at every count (32x512 CQ2 at 12000 27.0
+// against 41.4, 24x2048 CQ2 95.8 against 240.5).
+constexpr int kFewWaves = 16;
+constexpr int kFewWork = 4096;
+bool few_pays(cq_matrix *const *ms, int n, int rows) {
+    if (n > kKernargJobs || rows <= 0) return false;
+    const CqStore &s0 = *ms[0]->st;
+    if (!mfma_geometry_supported(s0.width, s0.group)) return false;
+    long long out = 0;
+    for (int k = 0; k < n; ++k) {
+        if (!uses_lut(ms[k]) || !shares_tables(s0, *ms[k]->st)) return false;
+        out += ms[k]->out;
+    }
+    const long long sets = (out + 31) / 32;
+    return out > 0 && s0.groups * sets <= kFewWaves && (sets == 1 || rows * sets <= kFewWork);
+}
+
+int run_few(cq_matrix *const *ms, int n, float *const *dsts, const float *x, int rows, hipStream_t stream) {
+    const CqStore &s0 = *ms[0]->st;
+    LutLaunch a;
+    std::memset(&a, 0, sizeof a);
+    int out = 0;
+    for (int k = 0; k < n; ++k) {
+        if (ms[k]->out == 0) continue;
+        fill_job(a.jobs[a.njobs], ms[k], x, dsts[k], rows);
+        a.wg0[a.njobs++] = out;
+        out += ms[k]->out;
+    }
+    HIP_TRY(launch_lut_few(a, s0.width, out, stream), "lut few-rows launch");
+    for (int k = 0; k < n; ++k) ms[k]->st->prepared.store(true);
+    return CQ_OK;
+}
+
 int run_product(cq_matrix *const *ms, int n, float *const *dsts, const float *x, int rows, hipStream_t stream,
                 const Fuse *fz = nullptr, const TabOut *to = nullptr, int *built = nullptr) {
     const CqStore &s0 = *ms[0]->st;
     const int mode = uses_lut(ms[0]) ? kModeLut : kModeExact;
+    if (mode == kModeLut && !(fz && fz->any()) && few_pays(ms, n, rows))
+        return run_few(ms, n, dsts, x, rows, stream);
     if (mode == kModeLut && tab_pays(ms, n, rows)) return run_tab(ms, n, dsts, x, rows, stream, fz);
     if (mode == kModeLut && n <= kKernargJobs && mfma_geometry_supported(s0.width, s0.group) &&
         mfma_pays(ms, n, rows))
@@ -1216,6 +1262,7 @@ const char *cq_gemm_path(const cq_matrix *m, int rows) {
     cq_matrix *mm = const_cast<cq_matrix *>(m);
     if (m && m->dense && dense_pays(&mm, 1, rows)) return "dense-f32";
     if (!m || !uses_lut(m)) return "nibble4";
+    if (few_pays(&mm, 1, rows)) return "lut";
     if (tab_pays(&mm, 1, rows)) return "lut-mfma-tab";
     if (mfma_geometry_supported(m->st->width, m->st->group) && mfma_pays(&mm, 1, rows)) return "lut-mfma";
     if (split_pays(&mm, 1, rows)) return "lut-mfma-split";

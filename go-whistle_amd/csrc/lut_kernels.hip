@@ -1068,7 +1068,170 @@ hipError_t launch_t(const LutLaunch &a, int waves, int gx, int gy, size_t lds, h
     return hipGetLastError();
 }
 
+// The lut product of few rows (jobs that share their tables): the mHC phi
+// products, 4 + 4 + lanes^2 rows of lanes * dim inputs, a narrow K
+// projection. For so few rows the tables are the work (16 entries a position
+// against one lookup a row), so none are built: a lane evaluates the entries
+// its row asks for, v = RNE(cb[code] x) (lut.go:239-282), and adds them as
+// float32 integers (below 2^21, exact in any order). A workgroup per
+// activation; wavefront s * groups + g takes rows 32 s .. 32 s + 31 of the
+// jobs' rows over group g, lane l row 32 s + l % 32 on half l / 32 of the
+// group's positions. The values come from LDS (a broadcast read a half), the
+// levels from a 16-entry table in LDS; the groups' terms meet in LDS and are
+// folded in group order (lut.go:297-310). Bit for bit the lut kernel's
+// result. Two or four activations a workgroup, sharing the levels' reads,
+// spilled at 16 wavefronts and were 2-5 times slower.
+//
+// What bounds it: latency at few activations (the index and value loads, the
+// rotation, 64 evaluations a lane, the fold), then VALU (a nibble takes 5
+// operations at 4 bits: shift, mask, multiply, round, add). Measured on MI355X
+// (graph-replayed, against the forms with tables): the phi products 4 + 4 +
+// 16 x 2048 CQ4 at 1, 375 and 12,000 activations 9.4, 38.0, 1,127 -> 5.5, 8.3,
+// 122 us; stacked as 24 x 2048 8.9, 21.3, 380 -> 5.2, 7.8, 118 us; 96 x 512 CQ4
+// at 1 and 375 5.7, 8.0 -> 5.2, 6.7 us.
+template <int BITS>
+__global__ __launch_bounds__(1024) void lut_few_kernel(LutLaunch a) {
+    constexpr int G = 128, NW = BITS == 4 ? 8 : 4;  // index words of a lane's half group
+    __shared__ __align__(16) float xs[16][G];  // scaled rotated groups
+    __shared__ float steps[16];
+    __shared__ float terms[16][32];  // [wavefront][row]
+    __shared__ float2 lvl[16];       // 4 bits: {cb[code], unused}; 2 bits: the pair's {cb[lo], cb[hi]}
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int groups = a.jobs[0].groups, in = a.jobs[0].in, units = a.jobs[0].units;
+    const int set = w / groups, g = w - set * groups, r = set * 32 + (lane & 31), t = blockIdx.x;
+
+    // the lane's row: its job's fields (uniform loads, selected)
+    const uint8_t *idx = a.jobs[0].idx;
+    const uint16_t *nrm = a.jobs[0].norm;
+    float *y = a.jobs[0].y;
+    long long ys = a.jobs[0].y_stride;
+    int rr = r, row0 = a.jobs[0].row0, out = a.jobs[0].out;
+#pragma unroll
+    for (int k = 1; k < kKernargJobs; ++k)
+        if (k < a.njobs && r >= a.wg0[k]) {
+            idx = a.jobs[k].idx;
+            nrm = a.jobs[k].norm;
+            y = a.jobs[k].y;
+            ys = a.jobs[k].y_stride;
+            rr = r - a.wg0[k];
+            row0 = a.jobs[k].row0;
+            out = a.jobs[k].out;
+        }
+    const bool real = rr < out;  // lanes past the last row repeat its index bytes, unused
+    const int root = row0 + (real ? rr : out - 1);
+    const size_t blk = root >> 6, ln = root & 63;
+    uint32_t iw[NW];
+#pragma unroll
+    for (int u = 0; u < NW / 4; ++u) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(
+            idx + ((blk * units + (g * 2 + half) * (NW / 4) + u) * 64 + ln) * 16);
+        iw[4 * u] = v.x;
+        iw[4 * u + 1] = v.y;
+        iw[4 * u + 2] = v.z;
+        iw[4 * u + 3] = v.w;
+    }
+    const float n = __half2float(__ushort_as_half(nrm[(blk * groups + g) * 64 + ln]));
+    if (tid < 16) lvl[tid] = BITS == 4 ? make_float2(a.jobs[0].cb[tid], 0.0f)
+                                       : make_float2(a.jobs[0].cb[tid & 3], a.jobs[0].cb[tid >> 2]);
+
+    // The group's rotation (the plain FWHT in the reference's stage order,
+    // kernel.go:384-393), lane = values 2 lane and 2 lane + 1, then the
+    // bound and the scale (lut.go:158-178, 219-225).
+    if (set == 0) {
+        const CQ_GLOBAL float *x = gptr(a.jobs[0].x) + static_cast<long long>(t) * a.jobs[0].x_stride;
+        float v[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int col = g * G + 2 * lane + e;
+            const float xv = x[min(col, in - 1)];
+            v[e] = col < in ? xv : 0.0f;
+        }
+        {
+            const float p = v[0], q = v[1];
+            v[0] = p + q;
+            v[1] = p - q;
+        }
+#pragma unroll
+        for (int h = 1; h < 64; h <<= 1)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float p = xor_lane(v[e], h);
+                v[e] = (lane & h) ? p - v[e] : v[e] + p;
+            }
+        float mx = BITS == 4 ? go_max(fabsf(v[0]), fabsf(v[1])) : fabsf(v[0]) + fabsf(v[1]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) mx = go_max(mx, xor_lane(mx, off));
+        const float m = a.jobs[0].cb_max * go_max(0.0f, mx);
+        const float inv = m > 0.0f ? static_cast<float>(kLutQ) / m : 0.0f;
+        if (lane == 0) steps[g] = m * a.jobs[0].lut_step;
+        *reinterpret_cast<float2 *>(&xs[g][2 * lane]) = make_float2(resid_value(v[0] * inv), resid_value(v[1] * inv));
+    }
+    __syncthreads();
+
+    float acc = 0.0f;
+    const char *lv = reinterpret_cast<const char *>(lvl);
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {  // a word is 8 nibbles: 8 values at 4 bits, 16 at 2
+        constexpr int VPW = BITS == 4 ? 8 : 16;
+        float2 lev[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t off = (j == 0 ? iw[q] << 3 : iw[q] >> (4 * j - 3)) & 0x78u;
+            if (BITS == 4)
+                lev[j].x = *reinterpret_cast<const float *>(lv + off);
+            else
+                lev[j] = *reinterpret_cast<const float2 *>(lv + off);
+        }
+        const float4 *xp = reinterpret_cast<const float4 *>(&xs[g][half * 64 + q * VPW]);
+        float xv[VPW];
+#pragma unroll
+        for (int i = 0; i < VPW / 4; ++i) {
+            const float4 f = xp[i];
+            xv[4 * i] = f.x;
+            xv[4 * i + 1] = f.y;
+            xv[4 * i + 2] = f.z;
+            xv[4 * i + 3] = f.w;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (BITS == 4) {
+                acc = acc + rintf(lev[j].x * xv[j]);
+            } else {
+                const float l = lev[j].x * xv[2 * j], h = lev[j].y * xv[2 * j + 1];
+                acc = acc + rintf(l + h);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // a word's reads at a time
+    }
+    const float s = acc + xor_lane<32>(acc);  // integers: exact
+    const float coef = n * steps[g];
+    if (half == 0) terms[w][lane] = s * coef;
+    __syncthreads();
+    if (g == 0 && half == 0 && real) {  // the set's first wavefront folds, lane = row
+        float yv = 0.0f;
+        for (int gi = 0; gi < groups; ++gi) yv = yv + terms[w + gi][lane];
+        y[static_cast<long long>(t) * ys + rr] = yv;
+    }
+}
+
 }  // namespace
+
+// Jobs of one geometry (128-weight groups) and codebook over one input, out
+// rows in all, wg0[k] job k's first among them: groups * ceil(out / 32) <= 16.
+hipError_t launch_lut_few(const LutLaunch &a, int bits, int out, hipStream_t s) {
+    const int rows = a.jobs[0].rows, groups = a.jobs[0].groups;
+    const long long waves = static_cast<long long>(groups) * ((out + 31) / 32);
+    if (a.njobs <= 0 || rows <= 0 || out <= 0 || groups <= 0 || waves > 16) return hipErrorInvalidValue;
+    const dim3 grid(rows), block(64 * static_cast<unsigned>(waves));
+    if (bits == 4)
+        hipLaunchKernelGGL((lut_few_kernel<4>), grid, block, 0, s, a);
+    else if (bits == 2)
+        hipLaunchKernelGGL((lut_few_kernel<2>), grid, block, 0, s, a);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
+}
 
 size_t lut_lds_bytes(int bits, int group_bytes, int gc, int tb, int bpw) {
     (void)bits;

@@ -93,28 +93,67 @@ __global__ __launch_bounds__(1024) void qkv_prep_kernel(PrepArgs a) {
     if (lane == 0) s8[row * hk + hh] = sc;
 }
 
-// A row of dim values (a multiple of 256, at most 4096) by 256 threads:
-// thread t holds values t, t + 256, ... in registers and stores them in LDS
-// transposed for the mean square's four in-order partial sums
-// (zc_partial_t), which lanes 0-3 of wavefront 0 add. Returns the
-// partials' sum of squares in float64 to every thread through LDS
-// (norm.go:91-109).
+// A row of dim values (at most 4096) by 256 threads: thread t holds values
+// t, t + 256, ... in registers; their squares (exact in float64) go to LDS by
+// partial, [i mod 4][i / 4], and lanes 0-3 of wavefront 0 only add them, in
+// order, 16 reads ahead of the adds; a tail of dim mod 4 values follows in
+// partial 0 (norm.go:91-109). Returns the sum of squares to every thread.
+// The chain of dim / 4 dependent float64 adds bounds these kernels. With the
+// converts and squares in the chain as well (float squares staged, each lane
+// converting and squaring its values between the adds) RMSUnit of 2048 took
+// 7.2 us a launch of one row and 10.7 us for 375 rows, against 4.9 and 8.8 us
+// (MI355X, kernel trace).
 constexpr int kRowMax = 4096;
 
-__device__ __forceinline__ double row_square_sum(const float *row, int dim, float (&v)[kRowMax / 256], float *t,
+// Doubles from one partial's squares to the next: 16-byte reads of the four
+// lanes fall on different banks.
+__host__ __device__ constexpr int row_stride(int dim) { return ((dim >> 2) + 31) / 32 * 32 + 2; }
+size_t row_lds(int dim) { return (4 * static_cast<size_t>(row_stride(dim)) + 4) * sizeof(double); }
+
+__device__ __forceinline__ double row_square_sum(const float *row, int dim, float (&v)[kRowMax / 256], double *t,
                                                  double *sum_sh) {
     const int tid = threadIdx.x;
-    const int V = dim >> 8, q = dim >> 2, stride = q + 4;
+    const int q = dim >> 2, full = dim & ~3, stride = row_stride(dim);
 #pragma unroll
-    for (int e = 0; e < kRowMax / 256; ++e)
-        if (e < V) {
-            const int i = tid + 256 * e;
-            v[e] = row[i];
-            t[(i & 3) * stride + (i >> 2)] = v[e];
-        }
+    for (int e = 0; e < kRowMax / 256; ++e) v[e] = tid + 256 * e < dim ? row[tid + 256 * e] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < kRowMax / 256; ++e) {
+        const int i = tid + 256 * e;
+        const double d = v[e];
+        if (i < dim) t[i < full ? (i & 3) * stride + (i >> 2) : 4 * stride + (i - full)] = d * d;
+    }
     __syncthreads();
     double part = 0.0;
-    if (tid < 4) part = zc_partial_t(t, stride, q, tid);
+    if (tid < 4) {
+        const double2 *r = reinterpret_cast<const double2 *>(t + tid * stride);
+        int j = 0;
+        double2 a[8];
+        if (q >= 16) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) a[k] = r[k];
+            for (; j + 32 <= q; j += 16) {  // the next 16 squares' reads go out before this round's adds
+                double2 b[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) b[k] = r[j / 2 + 8 + k];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    part = part + a[k].x;
+                    part = part + a[k].y;
+                }
+#pragma unroll
+                for (int k = 0; k < 8; ++k) a[k] = b[k];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                part = part + a[k].x;
+                part = part + a[k].y;
+            }
+            j += 16;
+        }
+        for (; j < q; ++j) part = part + t[tid * stride + j];
+        if (tid == 0)
+            for (int i = full; i < dim; ++i) part = part + t[4 * stride + (i - full)];
+    }
     const double p1 = __shfl(part, 1), p2 = __shfl(part, 2), p3 = __shfl(part, 3);
     if (tid == 0) *sum_sh = ((part + p1) + p2) + p3;
     __syncthreads();
@@ -124,11 +163,11 @@ __device__ __forceinline__ double row_square_sum(const float *row, int dim, floa
 // h = resid + float32(s * ZCRMSNorm(y)) per row (resid may be h).
 __global__ __launch_bounds__(256) void norm_scaled_add_kernel(float *h, const float *resid, const float *y,
                                                               const float *gain, float s, int dim) {
-    __shared__ __align__(16) float t[4 * (kRowMax / 4 + 4)];
+    extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double sum_sh;
     const int r = blockIdx.x, tid = threadIdx.x;
     float v[kRowMax / 256];
-    const double sum = row_square_sum(y + static_cast<long long>(r) * dim, dim, v, t, &sum_sh);
+    const double sum = row_square_sum(y + static_cast<long long>(r) * dim, dim, v, reinterpret_cast<double *>(smem), &sum_sh);
     // zc_rms: float32(sqrt(float64(float32(s / dim) + 1e-6)))
     const float ms = static_cast<float>(sum / static_cast<double>(dim));
     const float e = ms + 1e-6f;
@@ -151,24 +190,22 @@ __global__ __launch_bounds__(256) void norm_scaled_add_kernel(float *h, const fl
 // one chunk of dim): the mHC phi products' int8 input (mhc.go:99-106,
 // linear.go:80-87).
 __global__ __launch_bounds__(256) void rms_unit_row_kernel(float *dst, const float *x, int dim, int quant) {
-    __shared__ __align__(16) float t[4 * (kRowMax / 4 + 4)];
+    extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double sum_sh;
     __shared__ float red[4];
     const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int V = dim >> 8;
     float v[kRowMax / 256];
-    const double sum = row_square_sum(x + static_cast<long long>(r) * dim, dim, v, t, &sum_sh);
+    const double sum = row_square_sum(x + static_cast<long long>(r) * dim, dim, v, reinterpret_cast<double *>(smem), &sum_sh);
     const float ms = static_cast<float>(sum / static_cast<double>(dim));
     const float e = ms + 1e-6f;
     const float inv = static_cast<float>(1.0 / sqrt(static_cast<double>(e)));
 #pragma unroll
-    for (int k = 0; k < kRowMax / 256; ++k)
-        if (k < V) v[k] = v[k] * inv;
+    for (int k = 0; k < kRowMax / 256; ++k) v[k] = v[k] * inv;
     if (quant) {  // QuantizeRow's bound with Go's NaN-keeping max, then code * scale
         float m = 0.0f;
 #pragma unroll
         for (int k = 0; k < kRowMax / 256; ++k)
-            if (k < V) m = go_max(m, fabsf(v[k]));
+            if (tid + 256 * k < dim) m = go_max(m, fabsf(v[k]));
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) m = go_max(m, __shfl_xor(m, off));
         if (lane == 0) red[wave] = m;
@@ -177,12 +214,12 @@ __global__ __launch_bounds__(256) void rms_unit_row_kernel(float *dst, const flo
         const float sc = m > 0.0f ? m / 127.0f : 1.0f;
 #pragma unroll
         for (int k = 0; k < kRowMax / 256; ++k)
-            if (k < V) v[k] = static_cast<float>(go_int8_code(rintf(v[k] / sc))) * sc;
+            if (tid + 256 * k < dim) v[k] = static_cast<float>(go_int8_code(rintf(v[k] / sc))) * sc;
     }
     float *out = dst + static_cast<long long>(r) * dim;
 #pragma unroll
     for (int k = 0; k < kRowMax / 256; ++k)
-        if (k < V) out[tid + 256 * k] = v[k];
+        if (tid + 256 * k < dim) out[tid + 256 * k] = v[k];
 }
 
 __global__ __launch_bounds__(256) void expand_lanes_kernel(float *stream, const float *x, int lanes, int dim,
@@ -245,17 +282,18 @@ hipError_t launch_qkv_prep(const PrepArgs &a, int batch, hipStream_t s) {
 }
 
 bool row_kernel_dim(int dim) { return dim > 0 && dim % 256 == 0 && dim <= kRowMax; }
+bool row_unit_dim(int dim) { return dim > 0 && dim <= kRowMax; }
 
 hipError_t launch_norm_scaled_add(float *h, const float *resid, const float *y, const float *gain, float sc, int rows,
                                   int dim, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(norm_scaled_add_kernel, dim3(rows), dim3(256), 0, s, h, resid, y, gain, sc, dim);
+    hipLaunchKernelGGL(norm_scaled_add_kernel, dim3(rows), dim3(256), row_lds(dim), s, h, resid, y, gain, sc, dim);
     return hipGetLastError();
 }
 
 hipError_t launch_rms_unit_row(float *dst, const float *x, int rows, int dim, int quant, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(rms_unit_row_kernel, dim3(rows), dim3(256), 0, s, dst, x, dim, quant);
+    hipLaunchKernelGGL(rms_unit_row_kernel, dim3(rows), dim3(256), row_lds(dim), s, dst, x, dim, quant);
     return hipGetLastError();
 }
 

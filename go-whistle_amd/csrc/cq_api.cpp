@@ -2117,7 +2117,7 @@ int nd_hadamard_mlp_dev(float *out, const float *x, int rows, int dim, int na, i
     h.cond_u = cond_u;
     h.p1 = p1;
     h.p2 = p2;
-    HIP_TRY(launch_hadamard_mlp(h, rows, static_cast<hipStream_t>(stream)), "HadamardMLP launch");
+    HIP_TRY(launch_hadamard_mlp(h, rows, device_info().cus, static_cast<hipStream_t>(stream)), "HadamardMLP launch");
     return CQ_OK;
 }
 

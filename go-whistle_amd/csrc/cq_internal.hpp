@@ -389,7 +389,7 @@ struct HadaArgs {
     const float *cond_v, *cond_u;
     const int32_t *p1, *p2;
 };
-hipError_t launch_hadamard_mlp(const HadaArgs &h, int rows, hipStream_t s);
+hipError_t launch_hadamard_mlp(const HadaArgs &h, int rows, int cus, hipStream_t s);
 bool hadamard_shape_ok(int na, int nb, int dim, int rank);
 
 // Manifold hyper-connections around a block (mhc_kernels.hip): streams of

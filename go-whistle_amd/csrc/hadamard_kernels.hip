@@ -1,6 +1,8 @@
 // gfx950 HadamardMLP: Whistle's Monarch FFN (internal/needle/hadamard.go:
-// 12-24, 172-310), one workgroup per row, one thread per element of the
-// n = na * nb mix, float32 throughout as the reference computes it:
+// 12-24, 172-310), float32 throughout as the reference computes it, a
+// wavefront per row on the fp32 matrix instruction (hadamard_wave_kernel) or,
+// for factors past 32 and few rows of factors that do not fill 16 x 16 tiles,
+// a workgroup per row with one thread per element of the n = na * nb mix:
 //
 //   cond = 1 + softmax(x @ cond_v) @ cond_u
 //   z1   = kron(d1 * x; w1a, w1b)[p1]
@@ -22,6 +24,7 @@ namespace {
 
 constexpr int kHadaMaxN = 1024;
 constexpr int kHadaMaxRank = 32;
+constexpr int kHadaWaveRows = 2048;  // rows past which any factors to 32 take the wavefront form
 
 // out[c] = (a^T Z b)[c] for c = tid < n, Z in zs; ys is scratch of n.
 __device__ __forceinline__ float kron_elem(const float *zs, float *ys, const float *a, const float *b, int na,
@@ -122,10 +125,351 @@ __global__ __launch_bounds__(kHadaMaxN) void hadamard_mlp_kernel(HadaArgs h) {
     if (tid < dim) out[tid] = h.d4[tid] * k;
 }
 
+// A stage's mix of one row on one wavefront, with the fp32 matrix instruction
+// v_mfma_f32_16x16x4 (TA x TB tiles of 16; lane = 16 q + c). Z comes in as the
+// A operand, lane's rows 16 ta + c, columns 4 TB q + s: Y = Z b runs over its
+// columns in that order. A result register r is row 16 ta + 4 q + r of Y, which
+// is the B operand of a^T Y as it lies when the sum over Y's rows takes them
+// as (ta, r) with row 16 ta + 4 q + r in lane group q: no exchange between the
+// two products. out: [k tile][l tile], register r of row 16 tk + 4 q + r,
+// column 16 tb + c.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int TA, int TB>
+struct Mix {
+    float a[TA][4 * TA];  // a[16 ta + 4 q + r][16 tk + c] at [tk][4 ta + r]
+    float b[TB][4 * TB];  // b[4 TB q + s][16 tb + c] at [tb][s]
+    __device__ __forceinline__ void load(const float *pa, const float *pb, int na, int nb, int q, int c) {
+#pragma unroll
+        for (int tk = 0; tk < TA; ++tk)
+#pragma unroll
+            for (int i = 0; i < 4 * TA; ++i) {
+                const int row = (i >> 2) * 16 + 4 * q + (i & 3), col = tk * 16 + c;
+                a[tk][i] = row < na && col < na ? pa[row * na + col] : 0.0f;
+            }
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+            for (int s = 0; s < 4 * TB; ++s) {
+                const int row = 4 * TB * q + s, col = tb * 16 + c;
+                b[tb][s] = row < nb && col < nb ? pb[row * nb + col] : 0.0f;
+            }
+    }
+    __device__ __forceinline__ void run(const float (&z)[TA][4 * TB], f32x4 (&out)[TA][TB]) const {
+        f32x4 y[TA][TB];
+#pragma unroll
+        for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) y[ta][tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 4 * TB; ++s)
+#pragma unroll
+            for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb)
+                    y[ta][tb] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[ta][s], b[tb][s], y[ta][tb], 0, 0, 0);
+#pragma unroll
+        for (int tk = 0; tk < TA; ++tk)
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) out[tk][tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4 * TA; ++i)
+#pragma unroll
+            for (int tk = 0; tk < TA; ++tk)
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb)
+                    out[tk][tb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tk][i], y[i >> 2][tb][i & 3], out[tk][tb], 0, 0, 0);
+    }
+};
+
+// HadamardMLP for factors of at most 32, a wavefront per row: the row's
+// values stay in registers in the A operand's order, the mixes run on the
+// matrix cores, and only the permutations go through LDS (the wavefront's
+// own, no barrier). A workgroup stages the conditioning weights in LDS once
+// (CL, where they fit; in the lanes' order, free of bank conflicts) and its
+// four wavefronts run rows in turn with the factors and the element vectors
+// in registers, so the weights (60 KiB at 16 x 32 and rank 8) are read once a
+// workgroup and behind one load latency instead of one a stage. FULL: na = 16
+// TA, nb = 16 TB, dim a multiple of 4 and every pointer 16-byte aligned, so
+// that a lane's 4 TB columns are float4s.
+// What bounds it: at few rows one row's latency (two load rounds, three pairs
+// of products, the float64 sigmoids), then VALU (the sigmoids' float64 and the
+// cross-lane sums). Measured on MI355X against the workgroup form (us): 16 x 32
+// of 512, rank 8, at 1, 375, 3000 and 12,000 rows 12.4, 16.9, 64.1, 212.9 ->
+// 9.9, 11.0, 20.2, 54.0; 32 x 32 of 1024, rank 16, 23.9, 40.3, 200.9, 761 ->
+// 22.9, 24.4, 59.6, 179; 16 x 16 of 256 11.4, 12.4, 33.5, 95.5 -> 6.1, 6.6,
+// 11.1, 28.7. Its sums are fused (2.4e-7 from the float64 form over rows of
+// 512, against 2.5e-7).
+template <int TA, int TB, bool FULL, bool CL>
+__global__ __launch_bounds__(256) void hadamard_wave_kernel(HadaArgs h, int rows) {
+    constexpr int S = 4 * TB, E = TA * S;  // a lane's elements of a row
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15;
+    const int na = FULL ? 16 * TA : h.na, nb = FULL ? 16 * TB : h.nb, n = na * nb, dim = h.dim, rank = h.rank;
+    float *zs = reinterpret_cast<float *>(smem) + w * (TA * TB * 256);
+    float *cvl = reinterpret_cast<float *>(smem) + 4 * TA * TB * 256;  // [rank / 8][E][2][64][4]
+    const int rc = (rank + 7) >> 3;
+    float *cul = cvl + static_cast<size_t>(rc) * E * 512;              // [rank][E / 4][64][4]
+
+    // element ta, s of the lane: index (16 ta + c) nb + 4 TB q + s of the mix
+    auto index = [&](int ta, int s) { return (16 * ta + c) * nb + S * q + s; };
+    auto inside = [&](int ta, int s) { return FULL || (16 * ta + c < na && S * q + s < nb); };
+    auto gather4 = [&](const float *p, int ta, int s, int lim) -> float4 {  // elements s .. s + 3, zero from lim on
+        if constexpr (FULL) {
+            const int e = index(ta, s);
+            return e < lim ? *reinterpret_cast<const float4 *>(p + e) : make_float4(0, 0, 0, 0);
+        } else {
+            float f[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int e = index(ta, s + k);
+                f[k] = inside(ta, s + k) && e < lim ? p[e] : 0.0f;
+            }
+            return make_float4(f[0], f[1], f[2], f[3]);
+        }
+    };
+    auto gather = [&](float (&d)[TA][S], const float *p, int lim) {
+#pragma unroll
+        for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+            for (int s = 0; s < S; s += 4) {
+                const float4 f = gather4(p, ta, s, lim);
+                d[ta][s] = f.x;
+                d[ta][s + 1] = f.y;
+                d[ta][s + 2] = f.z;
+                d[ta][s + 3] = f.w;
+            }
+    };
+    // eight conditioning weights of an element, ranks 8 k0 ..
+    auto cond8 = [&](int ta, int s, int k0, float4 &f0, float4 &f1) {
+        const int e = index(ta, s);
+        f0 = f1 = make_float4(0, 0, 0, 0);
+        if (!inside(ta, s) || e >= dim) return;
+        const float *p = h.cond_v + static_cast<long long>(e) * rank + 8 * k0;
+        if (FULL && (rank & 7) == 0) {
+            f0 = *reinterpret_cast<const float4 *>(p);
+            f1 = *reinterpret_cast<const float4 *>(p + 4);
+        } else {
+            float v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = 8 * k0 + k < rank ? p[k] : 0.0f;
+            f0 = make_float4(v[0], v[1], v[2], v[3]);
+            f1 = make_float4(v[4], v[5], v[6], v[7]);
+        }
+    };
+
+    int row = blockIdx.x * 4 + w;
+    float xv[TA][S], d1[TA][S], d2[TA][S], b2[TA][S], d3[TA][S], d4[TA][TB][4];
+    int p1[TA][S], p2[TA][S];
+    gather(xv, h.x + static_cast<long long>(min(row, rows - 1)) * dim, dim);
+    gather(d1, h.d1, n);
+    Mix<TA, TB> m1, m2, m3;
+    m1.load(h.w1a, h.w1b, na, nb, q, c);
+    if constexpr (CL) {
+        for (int k0 = 0; k0 < rc; ++k0)
+            for (int i = w; i < E; i += 4) {
+                float4 f0, f1;
+                cond8(i / S, i % S, k0, f0, f1);
+                float *d = cvl + ((k0 * E + i) * 2 * 64 + lane) * 4;
+                *reinterpret_cast<float4 *>(d) = f0;
+                *reinterpret_cast<float4 *>(d + 256) = f1;
+            }
+        for (int i = w; i < rank * (E / 4); i += 4) {
+            const int r = i / (E / 4), e4 = i - r * (E / 4);
+            *reinterpret_cast<float4 *>(cul + (i * 64 + lane) * 4) =
+                gather4(h.cond_u + static_cast<long long>(r) * n, e4 * 4 / S, e4 * 4 % S, n);
+        }
+    }
+    m2.load(h.w2a, h.w2b, na, nb, q, c);
+    m3.load(h.w3a, h.w3b, na, nb, q, c);
+    gather(d2, h.d2, n);
+    gather(b2, h.b2, n);
+    gather(d3, h.d3, n);
+#pragma unroll
+    for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            p1[ta][s] = inside(ta, s) ? h.p1[index(ta, s)] : 0;
+            p2[ta][s] = inside(ta, s) ? h.p2[index(ta, s)] : 0;
+            if (static_cast<unsigned>(p1[ta][s]) >= static_cast<unsigned>(n)) p1[ta][s] = 0;  // a permutation of n
+            if (static_cast<unsigned>(p2[ta][s]) >= static_cast<unsigned>(n)) p2[ta][s] = 0;
+        }
+    auto result = [&](int tk, int tb, int r, int &e) {  // register r's index of the mix; false past the factors
+        const int k = 16 * tk + 4 * q + r, l = 16 * tb + c;
+        e = k * nb + l;
+        return FULL || (k < na && l < nb);
+    };
+#pragma unroll
+    for (int tk = 0; tk < TA; ++tk)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                int e;
+                d4[tk][tb][r] = result(tk, tb, r, e) ? h.d4[e] : 0.0f;
+            }
+    if constexpr (CL) __syncthreads();  // the only barrier: a wavefront is on its own from here
+
+    for (; row < rows; row += 4 * gridDim.x) {
+        const int next = min(row + 4 * static_cast<int>(gridDim.x), rows - 1);
+        float z[TA][S], xn[TA][S];
+        gather(xn, h.x + static_cast<long long>(next) * dim, dim);  // the next row's values, under this row's work
+#pragma unroll
+        for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+            for (int s = 0; s < S; ++s) z[ta][s] = d1[ta][s] * xv[ta][s];
+        f32x4 o[TA][TB];
+        m1.run(z, o);
+        auto to_lds = [&]() {
+#pragma unroll
+            for (int tk = 0; tk < TA; ++tk)
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        int e;
+                        if (result(tk, tb, r, e)) zs[e] = o[tk][tb][r];
+                    }
+        };
+        to_lds();
+
+        // cond = 1 + softmax(x cond_v) cond_u (hadamard.go:176-190): eight
+        // logits at a time, a lane's values then across the lanes; lane r
+        // keeps logit r.
+        float lg = -INFINITY;
+        for (int k0 = 0; k0 < rc; ++k0) {
+            float v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = 0.0f;
+#pragma unroll
+            for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    float4 f0, f1;
+                    if constexpr (CL) {
+                        const float *d = cvl + ((k0 * E + ta * S + s) * 2 * 64 + lane) * 4;
+                        f0 = *reinterpret_cast<const float4 *>(d);
+                        f1 = *reinterpret_cast<const float4 *>(d + 256);
+                    } else {
+                        cond8(ta, s, k0, f0, f1);
+                    }
+                    const float cv[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = fmaf(xv[ta][s], cv[k], v[k]);
+                }
+#pragma unroll
+            for (int hh = 1; hh < 64; hh <<= 1)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = v[k] + xor_lane(v[k], hh);
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (lane == 8 * k0 + k && lane < rank) lg = v[k];
+        }
+        float mx = lg;
+#pragma unroll
+        for (int hh = 32; hh > 0; hh >>= 1) mx = go_max(mx, xor_lane(mx, hh));
+        const float ex = lane < rank ? expf(lg - mx) : 0.0f;
+        float sum = ex;
+#pragma unroll
+        for (int hh = 1; hh < 64; hh <<= 1) sum = sum + xor_lane(sum, hh);
+        const float prob = ex / sum;
+        float cond[TA][S];
+#pragma unroll
+        for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+            for (int s = 0; s < S; ++s) cond[ta][s] = 0.0f;
+#pragma unroll 4
+        for (int r = 0; r < rank; ++r) {
+            const float p = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, prob), r));
+#pragma unroll
+            for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+                for (int s = 0; s < S; s += 4) {
+                    const float4 f = CL ? *reinterpret_cast<const float4 *>(cul + ((r * (E / 4) + (ta * S + s) / 4) * 64 + lane) * 4)
+                                        : gather4(h.cond_u + static_cast<long long>(r) * n, ta, s, n);
+                    cond[ta][s] = fmaf(p, f.x, cond[ta][s]);
+                    cond[ta][s + 1] = fmaf(p, f.y, cond[ta][s + 1]);
+                    cond[ta][s + 2] = fmaf(p, f.z, cond[ta][s + 2]);
+                    cond[ta][s + 3] = fmaf(p, f.w, cond[ta][s + 3]);
+                }
+        }
+
+        // z2's input: silu(d2 cond z1 + b2), z1 through p1
+#pragma unroll
+        for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const float t1 = d2[ta][s] * (cond[ta][s] + 1.0f);
+                const float a = t1 * zs[p1[ta][s]] + b2[ta][s];
+                z[ta][s] = inside(ta, s) ? a * gate_sigmoid(a) : 0.0f;
+            }
+        m2.run(z, o);
+        to_lds();
+#pragma unroll
+        for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+            for (int s = 0; s < S; ++s) z[ta][s] = inside(ta, s) ? d3[ta][s] * zs[p2[ta][s]] : 0.0f;
+        m3.run(z, o);
+        float *out = h.out + static_cast<long long>(row) * dim;
+#pragma unroll
+        for (int tk = 0; tk < TA; ++tk)
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    int e;
+                    if (result(tk, tb, r, e) && e < dim) out[e] = d4[tk][tb][r] * o[tk][tb][r];
+                }
+#pragma unroll
+        for (int ta = 0; ta < TA; ++ta)
+#pragma unroll
+            for (int s = 0; s < S; ++s) xv[ta][s] = xn[ta][s];
+    }
+}
+
+template <int TA, int TB, bool FULL, bool CL>
+hipError_t launch_wave_t(const HadaArgs &h, int rows, size_t lds, int cus, hipStream_t s) {
+    static std::atomic<unsigned long long> attr{0};
+    if (hipError_t e = lds_limit_once(reinterpret_cast<const void *>(&hadamard_wave_kernel<TA, TB, FULL, CL>), 160 * 1024, attr))
+        return e;
+    const int wgs = (rows + 3) / 4;  // four wavefronts, each a row at a time; two workgroups a CU at most
+    hipLaunchKernelGGL((hadamard_wave_kernel<TA, TB, FULL, CL>), dim3(wgs < 2 * cus ? wgs : 2 * cus), dim3(256), lds, s, h,
+                       rows);
+    return hipGetLastError();
+}
+
+template <int TA, int TB>
+hipError_t launch_wave(const HadaArgs &h, int rows, int cus, hipStream_t s, bool &taken) {
+    uintptr_t all = h.dim % 4 ? 1 : 0;
+    for (const void *p : {static_cast<const void *>(h.x), static_cast<const void *>(h.d1), static_cast<const void *>(h.d2),
+                          static_cast<const void *>(h.b2), static_cast<const void *>(h.d3),
+                          static_cast<const void *>(h.cond_v), static_cast<const void *>(h.cond_u)})
+        all |= reinterpret_cast<uintptr_t>(p);
+    const bool full = h.na == 16 * TA && h.nb == 16 * TB && (all & 15) == 0;
+    // Factors that do not fill their tiles load element by element, which
+    // costs few rows more than the workgroup form's barriers: 24 x 32 of 768 at
+    // 1, 375, 1500 and 3000 rows 31.3, 32.7, 63.2, 76.7 against 15.8, 23.3,
+    // 60.5, 118.7 us.
+    taken = full || rows > kHadaWaveRows;
+    if (!taken) return hipSuccess;
+    constexpr size_t zs = sizeof(float) * 4 * TA * TB * 256, elems = 4 * TA * TB;
+    const size_t lds = zs + sizeof(float) * elems * 64 * ((h.rank + 7) / 8 * 8 + h.rank);
+    const bool cl = lds <= 150 * 1024;  // the conditioning weights fit
+    if (full) return cl ? launch_wave_t<TA, TB, true, true>(h, rows, lds, cus, s) : launch_wave_t<TA, TB, true, false>(h, rows, zs, cus, s);
+    return cl ? launch_wave_t<TA, TB, false, true>(h, rows, lds, cus, s) : launch_wave_t<TA, TB, false, false>(h, rows, zs, cus, s);
+}
+
 }  // namespace
 
-hipError_t launch_hadamard_mlp(const HadaArgs &h, int rows, hipStream_t s) {
+hipError_t launch_hadamard_mlp(const HadaArgs &h, int rows, int cus, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
+    if (h.na <= 32 && h.nb <= 32) {
+        const int ta = (h.na + 15) / 16, tb = (h.nb + 15) / 16;
+        bool taken = false;
+        const hipError_t e = ta == 1 ? (tb == 1 ? launch_wave<1, 1>(h, rows, cus, s, taken) : launch_wave<1, 2>(h, rows, cus, s, taken))
+                                     : (tb == 1 ? launch_wave<2, 1>(h, rows, cus, s, taken) : launch_wave<2, 2>(h, rows, cus, s, taken));
+        if (taken || e != hipSuccess) return e;
+    }
     const int n = h.na * h.nb;
     const int threads = (n + 63) / 64 * 64;
     hipLaunchKernelGGL(hadamard_mlp_kernel, dim3(static_cast<unsigned>(rows)), dim3(threads), 0, s, h);

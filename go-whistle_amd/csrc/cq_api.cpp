@@ -1004,6 +1004,16 @@ int run_few(cq_matrix *const *ms, int n, float *const *dsts, const float *x, int
     return CQ_OK;
 }
 
+// Workgroups (four 64-row blocks by four activations) from which Exact's
+// products take the four-activation kernel: below it its two barriers a group
+// leave the chip idle where a workgroup per activation spreads wider. Measured
+// on MI355X (us, one activation against four): 2048x512 CQ4 at 32, 64 and 128
+// activations (64, 128, 256 workgroups) 10.5, 15.7, 22.5 against 13.7, 13.9,
+// 14.6; 16384x512 CQ4 at 5 and 16 (128, 256) 12.5, 21.6 against 18.0, 14.5;
+// 512x2048 CQ2 at 128 and 375 (64, 188) 19.7, 71.3 against 31.5, 39.2; 96x512
+// CQ4 at 375 (94) 9.6 against 17.8.
+constexpr long long kExactQuadWgs = 160;
+
 int run_product(cq_matrix *const *ms, int n, float *const *dsts, const float *x, int rows, hipStream_t stream,
                 const Fuse *fz = nullptr, const TabOut *to = nullptr, int *built = nullptr) {
     const CqStore &s0 = *ms[0]->st;
@@ -1036,7 +1046,15 @@ int run_product(cq_matrix *const *ms, int n, float *const *dsts, const float *x,
     LaunchPlan p = plan(s0, mode, nblk_total, rows);
     if (p.lds > device_info().max_lds)
         return fail(CQ_ERR_UNSUPPORTED, "cq: a product of group %d needs %zu bytes of LDS", s0.group, p.lds);
-    a.tb = p.tb;
+    bool quad = false;  // four activations a workgroup
+    if (mode == kModeExact && exact_quad_geometry(s0.group_bytes) && rows >= 4) {
+        long long wgs = 0;
+        for (int k = 0; k < n; ++k)
+            wgs += ((ms[k]->row0 + ms[k]->out + kBlockRows - 1) / kBlockRows - ms[k]->row0 / kBlockRows + 3) / 4;
+        wgs *= (rows + 3) / 4;
+        quad = wgs >= kExactQuadWgs;
+    }
+    a.tb = quad ? 4 : p.tb;
     a.gc = p.gc;
     int tiles = 0;
     a.nmats = 0;
@@ -1053,10 +1071,14 @@ int run_product(cq_matrix *const *ms, int n, float *const *dsts, const float *x,
         d.blk0 = m->row0 / kBlockRows;
         d.tile0 = tiles;
         const int nb = (m->row0 + m->out + kBlockRows - 1) / kBlockRows - d.blk0;
-        tiles += (nb + p.tb - 1) / p.tb;
+        tiles += (nb + a.tb - 1) / a.tb;
     }
     a.tiles = tiles;
     if (a.nmats == 0 || rows == 0) return CQ_OK;
+    if (quad) {
+        HIP_TRY(launch_exact_quad(a, s0.width, s0.group_bytes, stream), "exact product launch");
+        return CQ_OK;
+    }
     HIP_TRY(launch_product(a, s0.width, s0.group_bytes, mode, p.lds, stream), "product launch");
     if (mode == kModeLut)
         for (int k = 0; k < n; ++k) ms[k]->st->prepared.store(true);

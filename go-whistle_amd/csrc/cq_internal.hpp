@@ -72,6 +72,10 @@ struct ProdArgs {
 // bits, group_bytes select the template; mode is kModeLut or kModeExact.
 hipError_t launch_product(const ProdArgs &a, int bits, int group_bytes, int mode, size_t lds_bytes,
                           hipStream_t stream);
+// Exact's product of four activations at a time (a.tb = 4: tiles of four
+// blocks; groups of 8 to 64 index bytes).
+bool exact_quad_geometry(int group_bytes);
+hipError_t launch_exact_quad(const ProdArgs &a, int bits, int group_bytes, hipStream_t s);
 // LDS bytes per group of a chunk, and the fixed part, for choosing gc.
 size_t product_lds_bytes(int bits, int group_bytes, int mode, int gc, int tb);
 

@@ -15,7 +15,8 @@
 //              activations of a GEMM, lookupNibble's eight partial sums and
 //              tree; bit for bit the reference's.
 //
-// Work split. A workgroup (4 wavefronts) owns a tile of up to 4 blocks of
+// Work split of product_kernel (exact_quad_kernel, below, runs Exact's
+// products of many activations). A workgroup (4 wavefronts) owns a tile of up to 4 blocks of
 // 64 rows for one activation; each lane owns one row. Per chunk of groups
 // that fits LDS it rotates the activation, builds that chunk's tables in
 // LDS, and each wavefront takes (block, group) items: it streams the
@@ -354,6 +355,245 @@ hipError_t launch_one(const ProdArgs &a, size_t lds, hipStream_t stream) {
     return hipSuccess;
 }
 
+// m & byte B of t, in one VALU op (an SDWA byte select).
+template <int B>
+__device__ __forceinline__ uint32_t sdwa_and(uint32_t m, uint32_t t) {
+    uint32_t r;
+    if constexpr (B == 0)
+        asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0" : "=v"(r) : "v"(m), "v"(t));
+    else if constexpr (B == 1)
+        asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(r) : "v"(m), "v"(t));
+    else if constexpr (B == 2)
+        asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(r) : "v"(m), "v"(t));
+    else
+        asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3" : "=v"(r) : "v"(m), "v"(t));
+    return r;
+}
+__device__ __forceinline__ uint32_t sdwa_and(int b, uint32_t m, uint32_t t) {  // b a constant once loops unroll
+    switch (b) {
+        case 0: return sdwa_and<0>(m, t);
+        case 1: return sdwa_and<1>(m, t);
+        case 2: return sdwa_and<2>(m, t);
+        default: return sdwa_and<3>(m, t);
+    }
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Exact's products of four activations at a time (kernel.go:170-183, 239-374),
+// bit for bit product_kernel's. A workgroup takes four activations and up to
+// four 64-row blocks, one a wavefront (lane = row). Per group wavefront w
+// rotates activation w in registers; the tables hold the four activations'
+// entries side by side, [table][code][4], so one index nibble costs one
+// masked byte and one 16-byte LDS read (a code's 16 entries lie on distinct
+// banks) for four adds, where a table per activation cost a shift, a mask, an
+// address and a read per add. The next group's values, index units and norms
+// are loaded under the lookups. The last rows % 4 activations of a call take
+// lookupNibble's eight partial sums and tree.
+//
+// VALU-bound (product_kernel issued 4.8 operations a lookup and ran the VALU
+// 97% of the time; here 1.3 of a lookup's are the add and its share of the
+// index, the rest the tables and the rotation). Measured on MI355X, against a
+// workgroup per activation: 2048x512 CQ4 at 375 and 1500 activations 55.5,
+// 194.4 -> 25.8, 75.3 us, CQ2 31.5, 105.2 -> 16.0, 45.6 us; 16384x512 CQ4 at
+// 375 387.5 -> 138.5 us; 512x2048 CQ2 at 375 and 1500 71.3, 274 -> 39.2, 50.2
+// us.
+template <int BITS, int GB>
+__global__ __launch_bounds__(256) void exact_quad_kernel(ProdArgs a) {
+    using Gm = Geo<BITS, GB>;
+    constexpr int G = Gm::G, U = Gm::U, UPG = Gm::UPG, NT = Gm::NT;
+    constexpr int E = G >= 64 ? G / 64 : 1;  // a lane's values of a group
+    __shared__ __align__(16) f32x4 tab[NT * 16];
+    __shared__ __align__(16) float xh[G * 4];  // [position][activation]
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int act0 = blockIdx.y * 4, nact = min(4, a.rows - act0), tile = blockIdx.x;
+    const bool nib4 = act0 < a.nib4_rows;  // a multiple of 4: all four or none
+
+    const uint8_t *idx = a.mats[0].idx;
+    const uint16_t *nrm = a.mats[0].norm;
+    float *y = a.mats[0].y;
+    long long ys = a.mats[0].y_stride;
+    int row0 = a.mats[0].row0, out = a.mats[0].out, blk0 = a.mats[0].blk0, tile0 = 0;
+#pragma unroll
+    for (int k = 1; k < kMaxMatrices; ++k) {
+        if (k < a.nmats && tile >= a.mats[k].tile0) {
+            idx = a.mats[k].idx; nrm = a.mats[k].norm; y = a.mats[k].y; ys = a.mats[k].y_stride;
+            row0 = a.mats[k].row0; out = a.mats[k].out; blk0 = a.mats[k].blk0; tile0 = a.mats[k].tile0;
+        }
+    }
+    const int groups = a.groups, units = a.row_bytes / U, in = a.in;
+    const int blkEnd = (row0 + out + kBlockRows - 1) / kBlockRows;
+    const int mine = blk0 + (tile - tile0) * 4 + w, blk = min(mine, blkEnd - 1);  // past the view: the last block, unused
+    const float *x = a.x + static_cast<long long>(act0 + min(w, nact - 1)) * a.x_stride;
+    float cbl = a.cb[0], cbh = a.cb[0];  // the lane's code's level(s): a table entry is always of code lane % 16
+#pragma unroll
+    for (int c = 1; c < 16; ++c) {
+        if (BITS == 4 ? (lane & 15) == c : (lane & 3) == c) cbl = a.cb[c];
+        if (BITS == 2 && ((lane >> 2) & 3) == c) cbh = a.cb[c];
+    }
+
+    float xv[E];
+    uint32_t iw[UPG][4];
+    float n;
+    auto load_x = [&](int g) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int col = g * G + e * 64 + lane;
+            const bool ok = col < in && (G >= 64 || lane < G);
+            const float v = x[ok ? col : 0];
+            xv[e] = ok ? v : 0.0f;
+        }
+    };
+    auto load_idx = [&](int g) {
+        const uint8_t *up = idx + (static_cast<size_t>(blk) * units + static_cast<size_t>(g) * UPG) * 64 * U + lane * U;
+#pragma unroll
+        for (int u = 0; u < UPG; ++u) {
+            if constexpr (U == 16) {
+                const uint4 v = *reinterpret_cast<const uint4 *>(up + u * 64 * U);
+                iw[u][0] = v.x; iw[u][1] = v.y; iw[u][2] = v.z; iw[u][3] = v.w;
+            } else {
+                load_unit<U>(up + u * 64 * U, iw[u]);
+            }
+        }
+        n = half_bits_to_float(nrm[(static_cast<size_t>(blk) * groups + g) * 64 + lane]);
+    };
+    load_x(0);
+    load_idx(0);
+
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int g = 0; g < groups; ++g) {
+        // rotate (kernel.go:203-217): the plain FWHT, then 1/sqrt(G)
+#pragma unroll
+        for (int h = 1; h < (G < 64 ? G : 64); h <<= 1)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const float p = xor_lane(xv[e], h);
+                xv[e] = (lane & h) ? p - xv[e] : xv[e] + p;
+            }
+#pragma unroll
+        for (int h = 1; h < E; h <<= 1)
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                if (!(e & h)) {
+                    const float p = xv[e], q = xv[e | h];
+                    xv[e] = p + q;
+                    xv[e | h] = p - q;
+                }
+        if (G >= 64 || lane < G) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) xh[(e * 64 + lane) * 4 + w] = xv[e] * a.inv_sqrt;
+        }
+        __syncthreads();  // xh whole; every wavefront is done with the last group's tables
+        // nibbleTables (kernel.go:239-264): thread = code tid % 16 of tables tid / 16, tid / 16 + 16, ...
+#pragma unroll 4
+        for (int t = tid >> 4; t < NT; t += 16) {
+            f32x4 e;
+            if constexpr (BITS == 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(xh + 4 * t);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) e[k] = cbl * v[k];
+            } else {
+                const f32x4 v0 = *reinterpret_cast<const f32x4 *>(xh + 8 * t), v1 = *reinterpret_cast<const f32x4 *>(xh + 8 * t + 4);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float hb = cbh * v1[k], la = cbl * v0[k];
+                    e[k] = la + hb;
+                }
+            }
+            tab[t * 16 + (tid & 15)] = e;
+        }
+        __syncthreads();
+        uint32_t cw[UPG][4];
+#pragma unroll
+        for (int u = 0; u < UPG; ++u)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) cw[u][k] = iw[u][k];
+        const float cn = n;
+        if (g + 1 < groups) {
+            load_x(g + 1);
+            load_idx(g + 1);
+        }
+        const char *tb = reinterpret_cast<const char *>(tab);
+        auto entry = [&](int t, uint32_t off) { return *reinterpret_cast<const f32x4 *>(tb + t * 256 + off); };
+        if (nib4) {  // lookupNibble4 (kernel.go:330-374)
+            f32x4 fa = {0, 0, 0, 0}, fb = {0, 0, 0, 0};
+#pragma unroll
+            for (int u = 0; u < UPG; ++u)
+#pragma unroll
+                for (int q = 0; q < (U + 3) / 4; ++q) {
+                    const uint32_t hi = cw[u][q], lo = hi << 4;
+                    f32x4 el[4], eh[4];
+#pragma unroll
+                    for (int b = 0; b < (U < 4 ? U : 4); ++b) {
+                        const int t = 2 * (u * U + q * 4 + b);
+                        el[b] = entry(t, sdwa_and(b, 0xf0u, lo));
+                        eh[b] = entry(t + 1, sdwa_and(b, 0xf0u, hi));
+                    }
+#pragma unroll
+                    for (int b = 0; b < (U < 4 ? U : 4); ++b)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            fa[k] = fa[k] + el[b][k];
+                            fb[k] = fb[k] + eh[b][k];
+                        }
+                }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float ab = fa[k] + fb[k];
+                const float t = ab * cn;
+                acc[k] = acc[k] + t;
+            }
+        } else {  // lookupNibble (kernel.go:271-309)
+            f32x4 pa[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) pa[k] = f32x4{0, 0, 0, 0};
+#pragma unroll
+            for (int u = 0; u < UPG; ++u)
+#pragma unroll
+                for (int wd = 0; wd < U / 8; ++wd) {
+                    const uint32_t wl = cw[u][2 * wd], wh = cw[u][2 * wd + 1];
+                    const int t0 = 2 * u * U + wd * 16;
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const f32x4 e0 = entry(t0 + k, ((wl >> (4 * k)) & 15u) << 4), e1 = entry(t0 + k + 8, ((wh >> (4 * k)) & 15u) << 4);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const float pair = e0[j] + e1[j];
+                            pa[k][j] = pa[k][j] + pair;
+                        }
+                    }
+                }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float t01 = pa[0][j] + pa[1][j], t23 = pa[2][j] + pa[3][j], t45 = pa[4][j] + pa[5][j], t67 = pa[6][j] + pa[7][j];
+                const float t03 = t01 + t23, t47 = t45 + t67;
+                const float tt = t03 + t47;
+                const float t = tt * cn;
+                acc[j] = acc[j] + t;
+            }
+        }
+    }
+    const int r = blk * kBlockRows + lane;
+    if (mine < blkEnd && r >= row0 && r < row0 + out)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k < nact) y[static_cast<long long>(act0 + k) * ys + (r - row0)] = acc[k];
+}
+
+template <int BITS, int GB>
+hipError_t launch_quad(const ProdArgs &a, hipStream_t stream) {
+    for (int r0 = 0; r0 < a.rows; r0 += 4 * 65535) {
+        ProdArgs b = a;
+        b.rows = min(4 * 65535, a.rows - r0);
+        b.x = a.x + static_cast<long long>(r0) * a.x_stride;
+        b.nib4_rows = a.nib4_rows - r0;
+        for (int k = 0; k < a.nmats; ++k) b.mats[k].y = a.mats[k].y + static_cast<long long>(r0) * a.mats[k].y_stride;
+        hipLaunchKernelGGL((exact_quad_kernel<BITS, GB>), dim3(a.tiles, (b.rows + 3) / 4), dim3(256), 0, stream, b);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
+}
+
 template <int MODE>
 hipError_t dispatch(const ProdArgs &a, int bits, int gb, size_t lds, hipStream_t s) {
     if (bits == 4) {
@@ -438,6 +678,24 @@ hipError_t launch_product(const ProdArgs &a, int bits, int group_bytes, int mode
     if (a.rows <= 0 || a.tiles <= 0) return hipSuccess;
     return mode == kModeLut ? dispatch<kModeLut>(a, bits, group_bytes, lds, stream)
                             : dispatch<kModeExact>(a, bits, group_bytes, lds, stream);
+}
+
+bool exact_quad_geometry(int group_bytes) { return group_bytes >= 8 && group_bytes <= 64; }
+
+hipError_t launch_exact_quad(const ProdArgs &a, int bits, int group_bytes, hipStream_t s) {
+    if (a.rows <= 0 || a.tiles <= 0) return hipSuccess;
+    if (a.tb != 4) return hipErrorInvalidValue;
+    switch (bits * 256 + group_bytes) {
+        case 4 * 256 + 8: return launch_quad<4, 8>(a, s);
+        case 4 * 256 + 16: return launch_quad<4, 16>(a, s);
+        case 4 * 256 + 32: return launch_quad<4, 32>(a, s);
+        case 4 * 256 + 64: return launch_quad<4, 64>(a, s);
+        case 2 * 256 + 8: return launch_quad<2, 8>(a, s);
+        case 2 * 256 + 16: return launch_quad<2, 16>(a, s);
+        case 2 * 256 + 32: return launch_quad<2, 32>(a, s);
+        case 2 * 256 + 64: return launch_quad<2, 64>(a, s);
+    }
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_rows(const RowArgs &a, hipStream_t stream) {

@@ -1927,7 +1927,7 @@ static int attend_impl(float *out, long long out_stride, const float *q, long lo
     AttendArgs a{out, out_stride, q, q_stride, t, heads, kq, ks, k_cols, qk, vq, vs, v_cols, vd,
                  kv_stride, s_stride, spans, nk_max, vchunk, resident, scale, quant_q, batch,
                  rope_cos, rope_sin, qpos, kv_index, kv_streams, pages, page_stride, page_shift, pool_pages};
-    HIP_TRY(launch_attend_int8(a, static_cast<hipStream_t>(stream)), "attend launch");
+    HIP_TRY(launch_attend_int8(a, device_info().cus, static_cast<hipStream_t>(stream)), "attend launch");
     return CQ_OK;
 }
 

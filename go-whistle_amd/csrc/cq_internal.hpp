@@ -347,7 +347,7 @@ struct AttendArgs {
     int page_stride, page_shift, pool_pages;
     int page_lds;  // set by the launcher: the byte offset of the LDS copy of the page table
 };
-hipError_t launch_attend_int8(const AttendArgs &a, hipStream_t stream);
+hipError_t launch_attend_int8(const AttendArgs &a, int cus, hipStream_t stream);
 constexpr int kAttendMaxPages = 1024;  // a paged launch's pages per stream
 
 // The cache stream a workgroup of stream b reads (kv_index, or b itself),

@@ -1493,6 +1493,260 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
     outp[lane] = acc;
 }
 
+// AttendInt8Spans for prompts: many query rows over one cache (t > 1, value
+// heads of 64 codes, key heads of at most 64). A workgroup takes 4 to 16
+// (query row, head) pairs of one stream and key head, one a wavefront, and
+// stages the codes and scales of the keys that any of them sees in LDS once:
+// a cache row is read once a workgroup instead of once a pair, and after the
+// staging no wavefront waits on memory. A wavefront runs its pair alone: the
+// query (quantised as asked), the logits a key per lane, the softmax (amd64's
+// expSubSum), then lane d the in-order chain of output d. The values are
+// staged as fp16 (every int8 code is one), two keys to a word, so that a key
+// and output costs a mixed multiply and an add with no convert. Same
+// arithmetic as attend_kernel.
+//
+// Bound by VALU issue (1,667 instructions a pair of 448 keys, busy 61% of the
+// kernel) behind one exposed staging. Measured on MI355X, 8 heads of 64, 448
+// keys a stream, causal, against a wavefront a pair reading its own rows:
+// 4 streams x 96 rows, 2 key heads of 48 codes 31.5 -> 20.8 us (int8 values,
+// converted by each pair, 21.9); 8 key heads of 64 32.3 -> 18.3; 16 streams x
+// 32 rows 36.0 -> 23.2 (8 key heads 43.7 -> 24.0); 64 streams x 2 rows
+// 20.8 -> 18.0. Loading a thread's whole share before its first store, the
+// query's with it: 21.5 (92 registers for 60).
+constexpr int kRowsMaxWaves = 16;
+
+using half2v = __attribute__((ext_vector_type(2))) _Float16;
+using half8v = __attribute__((ext_vector_type(8))) _Float16;
+
+// Bytes between staged key rows: 16-byte reads of 16 lanes on distinct banks.
+__host__ __device__ constexpr int rows_key_stride(int qk) { return qk % 32 == 0 ? qk + 16 : qk; }
+
+__global__ __launch_bounds__(64 * kRowsMaxWaves) void attend_rows_kernel(AttendArgs a, int per_group) {
+    constexpr int VD = 64;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int lo_sh[kRowsMaxWaves], hi_sh[kRowsMaxWaves];
+    __shared__ __align__(16) int8_t q8s[kRowsMaxWaves][64];
+    __shared__ __align__(16) float qfs[kRowsMaxWaves][64];
+    const int tid = threadIdx.x, lane = tid & 63, nw = blockDim.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kv_heads = a.k_cols / a.qk, rep = a.heads / kv_heads, pairs = a.t * rep;
+    const int grp = blockIdx.x % per_group, bk = blockIdx.x / per_group;
+    const int b = bk / kv_heads, kv = bk % kv_heads;
+    const int p = grp * nw + w;
+    const bool live = p < pairs;
+    const int i = live ? p / rep : a.t - 1, h = kv * rep + (live ? p % rep : 0);
+    const long long kb = attend_cache_of(a, b);
+    if (kb < 0) return;  // no cache: the whole workgroup
+    const int32_t *sp = a.spans + (static_cast<long long>(b) * a.t + i) * 4;
+    const int lo0 = sp[0], len0 = sp[1] - sp[0], lo1 = sp[2], len1 = sp[3] - sp[2];
+    const int n = len0 + len1;
+    const bool off = lo0 < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max ||
+                     n > a.nk_max;
+    const bool run = live && !off;  // spans off the cache leave the output untouched
+    attend_stage_pages(a, b, smem);
+    const int32_t *pgs = reinterpret_cast<const int32_t *>(smem + a.page_lds);
+    if (lane == 0) {
+        int lo = INT_MAX, hi = 0;
+        if (run && len0 > 0) { lo = lo0; hi = sp[1]; }
+        if (run && len1 > 0) { lo = min(lo, lo1); hi = max(hi, sp[3]); }
+        lo_sh[w] = lo;
+        hi_sh[w] = hi;
+    }
+    const float *qi = a.q + b * a.q_stride + (static_cast<long long>(i) * a.heads + h) * a.qk;
+    const int qp = a.rope_cos ? a.qpos[static_cast<long long>(b) * a.t + i] : 0;
+    const float qv = lane < a.qk ? query_value(a, qi, qp, lane) : 0.0f;
+    __syncthreads();
+    int base = INT_MAX, end = 0;
+    for (int k = 0; k < nw; ++k) {
+        base = min(base, lo_sh[k]);
+        end = max(end, hi_sh[k]);
+    }
+    const int cnt = max(0, end - min(base, end));
+
+    const int kst = rows_key_stride(a.qk), nk4 = (a.nk_max + 3) & ~3;
+    float *s = reinterpret_cast<float *>(smem) + w * (nk4 + 8);
+    float *ksl = reinterpret_cast<float *>(smem) + nw * (nk4 + 8), *vsl = ksl + nk4;
+    half2v *vl = reinterpret_cast<half2v *>(vsl + nk4);                            // [key / 2][64]
+    int8_t *kl = reinterpret_cast<int8_t *>(vl + static_cast<size_t>(nk4 / 2) * VD);  // [key][kst]
+    {
+        const int8_t *kq = a.kq + kb * a.kv_stride + kv * a.qk, *vq = a.vq + kb * a.kv_stride + kv * VD;
+        const float *ks = a.ks + kb * a.s_stride + kv, *vs = a.vs + kb * a.s_stride + kv;
+        const int kp = a.qk / 16, nt = blockDim.x;
+        for (int e = tid; e < (cnt + 1) / 2 * 4; e += nt) {  // two value rows, 16 outputs
+            const int j = e >> 2 << 1, c = e & 3;
+            const int4 va = *reinterpret_cast<const int4 *>(vq + attend_row(a, pgs, base + j) * a.v_cols + c * 16);
+            const int4 vb = *reinterpret_cast<const int4 *>(vq + attend_row(a, pgs, base + min(j + 1, cnt - 1)) * a.v_cols + c * 16);
+            const int wa[4] = {va.x, va.y, va.z, va.w}, wb[4] = {vb.x, vb.y, vb.z, vb.w};
+            half2v *to = vl + (j >> 1) * VD + c * 16;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                half2v p[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    p[k] = half2v{static_cast<_Float16>(static_cast<int8_t>(wa[q] >> (8 * k))),
+                                  static_cast<_Float16>(static_cast<int8_t>(wb[q] >> (8 * k)))};
+                *reinterpret_cast<half8v *>(to + 4 * q) =
+                    half8v{p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y};
+            }
+        }
+        for (int e = tid; e < cnt * kp; e += nt) {
+            const int j = e / kp, c = e - j * kp;
+            *reinterpret_cast<int4 *>(kl + j * kst + c * 16) =
+                *reinterpret_cast<const int4 *>(kq + attend_row(a, pgs, base + j) * a.k_cols + c * 16);
+        }
+        for (int j = tid; j < cnt; j += nt) {
+            const long long row = attend_row(a, pgs, base + j);
+            ksl[j] = ks[row * kv_heads];
+            vsl[j] = vs[row * kv_heads];
+        }
+    }
+    // QuantizeRow of the query head (int8.go:226-228), while the codes land
+    float sq = 0.0f;
+    qfs[w][lane] = qv;
+    if (a.quant_q) {
+        float m = fabsf(qv);
+#pragma unroll
+        for (int hh = 32; hh > 0; hh >>= 1) m = go_max(m, xor_lane(m, hh));
+        sq = m > 0.0f ? m / 127.0f : 1.0f;
+        q8s[w][lane] = static_cast<int8_t>(go_int8_code(rintf(qv / sq)));
+    }
+    __syncthreads();  // the last barrier: a wavefront is on its own from here
+    if (!run) return;
+    float *outp = a.out + b * a.out_stride + (static_cast<long long>(i) * a.heads + h) * VD;
+    if (n == 0) {
+        outp[lane] = 0.0f;
+        return;
+    }
+
+    // Element j's place: shifted so that a span's weights lie as its keys do,
+    // modulo the four that one read takes.
+    const int k0 = lo0 - base, k1 = lo1 - base - len0;  // element j's key: k0 + j, k1 + j past len0
+    const int sh0 = k0 & 3, sh1 = sh0 + ((k1 - sh0) & 3);
+    auto at = [&](int j) { return j + (j < len0 ? sh0 : sh1); };
+    auto key_of = [&](int j) { return j + (j < len0 ? k0 : k1); };
+
+    // 1. Logits (int8Logits / dotsF32I8), a key per lane.
+    const int kp = a.qk / 16;
+    int4 qw[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (c < kp) qw[c] = *reinterpret_cast<const int4 *>(q8s[w] + 16 * c);
+    float mx = -INFINITY;
+    for (int j = lane; j < n; j += 64) {
+        const int key = key_of(j);
+        const int8_t *row = kl + key * kst;
+        const float sk = ksl[key];
+        float lg;
+        if (a.quant_q) {
+            int dot = 0;  // exact in any order
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (c < kp) {
+                    const int4 kw = *reinterpret_cast<const int4 *>(row + 16 * c);
+                    dot = __builtin_amdgcn_sdot4(kw.x, qw[c].x, dot, false);
+                    dot = __builtin_amdgcn_sdot4(kw.y, qw[c].y, dot, false);
+                    dot = __builtin_amdgcn_sdot4(kw.z, qw[c].z, dot, false);
+                    dot = __builtin_amdgcn_sdot4(kw.w, qw[c].w, dot, false);
+                }
+            const float scl = sq * sk;
+            const float t1 = static_cast<float>(dot) * scl;
+            lg = t1 / a.scale;
+        } else {
+            float dot = 0.0f;  // in order
+            for (int c = 0; c < kp; ++c) {
+                const int4 kw = *reinterpret_cast<const int4 *>(row + 16 * c);
+                const int cw[4] = {kw.x, kw.y, kw.z, kw.w};
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const float pr = qfs[w][16 * c + e] * static_cast<float>(static_cast<int8_t>(cw[e >> 2] >> (8 * (e & 3))));
+                    dot = dot + pr;
+                }
+            }
+            const float t1 = dot * sk;
+            lg = t1 / a.scale;
+        }
+        s[at(j)] = lg;
+        mx = go_max(mx, lg);
+    }
+
+    // 2. softmaxInPlace with amd64's expSubSum: eight lane sums of stride 8.
+#pragma unroll
+    for (int hh = 32; hh > 0; hh >>= 1) mx = go_max(mx, xor_lane(mx, hh));
+    const int n8 = n & ~7;
+    for (int j = lane; j < n; j += 64) s[at(j)] = j < n8 ? exp_lane(s[at(j)] - mx) : exp_generic(s[at(j)] - mx);
+    float acc8 = 0.0f;
+    if (lane < 8) {
+        int j = lane;
+        for (; j + 56 < n8; j += 64) {
+            float e[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) e[k] = s[at(j + 8 * k)];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc8 = acc8 + e[k];
+        }
+        for (; j < n8; j += 8) acc8 = acc8 + s[at(j)];
+    }
+    float sum;
+    if (n8 > 0) {  // (lo + hi), then the two pairwise adds
+        const float x = acc8 + xor_lane<4>(acc8);  // lanes 0-3: red[l] + red[l + 4]
+        const float hsum = x + xor_lane<1>(x);     // lanes 0, 2: x0 + x1, x2 + x3
+        sum = hsum + xor_lane<2>(hsum);
+        sum = __shfl(sum, 0);
+        if (n8 != n) {
+            float tail = 0.0f;
+            for (int j = n8; j < n; ++j) tail = tail + s[at(j)];
+            sum = sum + tail;
+        }
+    } else {
+        sum = 0.0f;
+        for (int j = 0; j < n; ++j) sum = sum + s[at(j)];
+    }
+    for (int j = lane; j < n; j += 64) {
+        const int key = key_of(j);
+        const float pr = s[at(j)] / sum;
+        s[at(j)] = pr * vsl[key];
+    }
+
+    // 3. axpysI8 (int8kernel.go:360-368): lane d's products in key order,
+    // span by span. fma(code, weight, 0) rounds as the product does (acc is
+    // never -0) and takes the fp16 code as it lies.
+    float acc = 0.0f;
+    for (int part = 0; part < 2; ++part) {
+        int key = part == 0 ? k0 : k1 + len0;
+        const int stop = key + (part == 0 ? len0 : len1);
+        const float *wt = s + (part == 0 ? sh0 - k0 : sh1 - k1);  // by key: 16-byte aligned where the key is a multiple of 4
+        auto one = [&](int k) {
+            const float pr = wt[k] * static_cast<float>(reinterpret_cast<const _Float16 *>(vl + (k >> 1) * VD + lane)[k & 1]);
+            acc = acc + pr;
+        };
+        for (; (key & 3) && key < stop; ++key) one(key);
+        for (; key + 32 <= stop; key += 32) {  // every read out before the first product
+            half2v c[16];
+            float4 wv[8];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) c[k] = vl[((key >> 1) + k) * VD + lane];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) wv[q] = *reinterpret_cast<const float4 *>(wt + key + 4 * q);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                acc = acc + fmaf(static_cast<float>(c[2 * q].x), wv[q].x, 0.0f);
+                acc = acc + fmaf(static_cast<float>(c[2 * q].y), wv[q].y, 0.0f);
+                acc = acc + fmaf(static_cast<float>(c[2 * q + 1].x), wv[q].z, 0.0f);
+                acc = acc + fmaf(static_cast<float>(c[2 * q + 1].y), wv[q].w, 0.0f);
+            }
+        }
+        for (; key < stop; ++key) one(key);
+    }
+    outp[lane] = acc;
+}
+
+// LDS of the prompt form with nw wavefronts, without a paged launch's table.
+size_t rows_lds(const AttendArgs &a, int nw) {
+    const size_t nk4 = (static_cast<size_t>(a.nk_max) + 3) & ~size_t(3);
+    return (nk4 + 8) * 4 * nw + nk4 * (8 + 2 * kChainVd + rows_key_stride(a.qk));
+}
+
 }  // namespace
 
 hipError_t launch_gather_rows(void *dst, const void *src, const int32_t *idx, const int32_t *len, int streams,
@@ -1606,7 +1860,7 @@ size_t chain_lds(const AttendArgs &a, int jc, int rs) {
 // The resident form also holds the two product buffers behind the rows.
 size_t chain_res_lds(const AttendArgs &a, int rs) { return chain_lds(a, 64, rs) + 2 * sizeof(float) * kProdFloats; }
 
-hipError_t launch_attend_int8(const AttendArgs &args, hipStream_t stream) {
+hipError_t launch_attend_int8(const AttendArgs &args, int cus, hipStream_t stream) {
     AttendArgs a = args;
     if (a.t <= 0 || a.heads <= 0 || a.batch <= 0) return hipSuccess;
     // A paged launch keeps the stream's page table behind the kernel's own
@@ -1627,6 +1881,27 @@ hipError_t launch_attend_int8(const AttendArgs &args, hipStream_t stream) {
             const int rs = std::max(1, (a.nk_max + 63) / 64);
             const size_t lds = with_pages(chain_res_lds(a, rs));
             if (lds <= 150 * 1024) return launch_attend_chain<4, 64, true>(a, rs, lds, stream);
+        }
+        // Prompts of more workgroups than stay resident: a workgroup of 4 to 16
+        // pairs, about one for each CU. Fewer than eight wavefronts need a CU
+        // each, or LDS for two workgroups on one: 128 streams x 4 rows of 8
+        // key heads took 65 us with four alone on a CU, 49.6 the way below.
+        if (a.t > 1) {
+            const int kv_heads = a.k_cols / a.qk, pairs = a.t * (a.heads / kv_heads);
+            const long long groups = static_cast<long long>(a.batch) * kv_heads, total = groups * pairs;
+            int nw = static_cast<int>(std::min<long long>(kRowsMaxWaves, std::max(4LL, (total + cus - 1) / cus)));
+            nw = std::min(nw, pairs);
+            while (nw > 4 && with_pages(rows_lds(a, nw)) > 150 * 1024) --nw;
+            const int per_group = (pairs + nw - 1) / nw;
+            const size_t lds = with_pages(rows_lds(a, nw));
+            const bool enough = nw >= 8 || groups * per_group <= cus || 2 * lds <= 150 * 1024;
+            if (nw >= 4 && enough && lds <= 150 * 1024 && groups * per_group <= INT_MAX) {
+                static std::atomic<unsigned long long> attr{0};
+                if (hipError_t e = lds_limit_once(reinterpret_cast<const void *>(&attend_rows_kernel), 152 * 1024, attr)) return e;
+                hipLaunchKernelGGL(attend_rows_kernel, dim3(static_cast<unsigned>(groups * per_group)), dim3(64 * nw), lds, stream,
+                                   a, per_group);
+                return hipGetLastError();
+            }
         }
         if (a.qk == kChainVd) {
             // many streams: key and value chunks through a ring of 6 slots

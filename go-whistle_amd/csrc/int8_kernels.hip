@@ -1227,6 +1227,7 @@ __device__ __forceinline__ void dma4(const void *src, unsigned lds) {
 }
 
 constexpr int kRingJc = 32;                     // keys per ring chunk
+constexpr int kRingSlots = 4;                   // ring slots: two read in a turn, two in flight
 constexpr int kRingSlot = kRingJc * 64 + kRingJc * 4;  // 64 codes per key, then the keys' scales
 
 // AttendInt8Spans for one (stream, query row, head) per single-wavefront
@@ -1234,14 +1235,23 @@ constexpr int kRingSlot = kRingJc * 64 + kRingJc * 4;  // 64 codes per key, then
 // many-stream form. Key chunks, then value chunks, of 32 keys stream through
 // one LDS ring of RS slots (global_load_lds, refilled behind the reads); a
 // slot holds the chunk's rows [key][64 codes] and the 32 keys' scales, so no
-// load of the kernel waits on its own: every wavefront keeps RS chunks of
-// HBM reads in flight.
-//   1. the query; the logits chunk by chunk, two lanes per key (exact int32
+// load of the kernel waits on its own: every wavefront keeps RS - 2 to RS
+// chunks of HBM reads in flight.
+//   1. the query; the logits two chunks a turn, a key per lane (exact int32
 //      dots, or the float32 query in order);
 //   2. the softmax (amd64's expSubSum) with the eight lane sums read at
 //      stride 8;
-//   3. per value chunk the keys' weights p_j * vscale_j, then lane d's
-//      in-order chain of fl(w_j * code_jd).
+//   3. two value chunks a turn: the keys' weights p_j * vscale_j, then lane
+//      d's in-order chain of fl(w_j * code_jd).
+// What bounds it: HBM over long caches; else a wavefront's own chain of LDS
+// reads, divisions and adds from chunk to chunk (halving the streams of the
+// 448-key call below takes 15% off it), so a turn takes two chunks: their
+// logits and weights pay that latency once, and a key per lane needs no lane
+// exchange. Measured on MI355X, 8 heads (one chunk a turn, two lanes a key, six
+// slots -> now): 256 streams of 1 to 448 keys 28.4 -> 25.5 us, of 1 to 128 13.4
+// -> 12.1, 128 streams 25.0 -> 21.4, 256 streams of 1 to 1500 keys 85 -> 77.
+// Slots 5, 6 and 8 instead of 4: 26.5, 26.7, 27.4 us and 79, 80, 84. The second
+// chunk's codes read between the first one's products: 27.2 us (146 registers).
 // Same arithmetic as attend_kernel.
 template <int RS>
 __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) {
@@ -1286,6 +1296,7 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
     float *s = reinterpret_cast<float *>(smem);  // logits, exponentials, then weights
     int8_t *ring = reinterpret_cast<int8_t *>(s + nk_pad);
     __shared__ float qf[ROW];
+    __shared__ __align__(16) int8_t q8[ROW];
     __shared__ float red[8];
 
     const float *qi = a.q + b * a.q_stride + (static_cast<long long>(i) * a.heads + h) * ROW;
@@ -1316,10 +1327,12 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
         const int key = key_of(j0 + (lane < cnt ? lane : 0));
         if (lane < JC) dma4(sc + attend_row(a, pgs, key) * kv_heads + kv, lds_offset(slot + JC * ROW));
     };
-    // Chunk g has landed: at most the chunks issued after it are in flight.
-    auto wait_chunk = [&](int g) {
-        if (g + RS - 1 < total) wait_vm_const<LPC * (RS - 1)>();
-        else wait_vm(LPC * (total - 1 - g));
+    // A turn takes chunk g, or g and g + 1, when chunks below g + RS have been
+    // issued (the refills are the earlier turns'): they have landed once only
+    // the chunks issued after the turn's last are in flight.
+    auto wait_turn = [&](int g, bool two) {
+        if (two && g + RS <= total) wait_vm_const<LPC * (RS - 2)>();
+        else wait_vm(LPC * (min(g + RS, total) - 1 - (two ? g + 1 : g)));
     };
     auto refill = [&](int g) {  // after chunk g's reads: chunk g + RS into its slot
         if (g + RS < total) {
@@ -1336,57 +1349,50 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
     for (int g = 0; g < min(RS, total); ++g) dma(g);
     qf[lane] = qv;
     float sq = 0.0f;
-    int4 q4[2];  // this lane's half of the int8 query (32 codes)
-    const int half = lane >> 5;
+    int4 q4[4];  // the int8 query in the lane's order of pieces
     if (a.quant_q) {
         float m = fabsf(qv);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) m = go_max(m, __shfl_xor(m, off));
         const float sc = m > 0.0f ? m / 127.0f : 1.0f;
-        const int code = go_int8_code(rintf(qv / sc)) & 255;
-        // gather this lane's 32 query codes (lanes 32*half ..) into 8 words
-        int words[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int c0 = __shfl(code, 32 * half + 4 * k), c1 = __shfl(code, 32 * half + 4 * k + 1);
-            const int c2 = __shfl(code, 32 * half + 4 * k + 2), c3 = __shfl(code, 32 * half + 4 * k + 3);
-            words[k] = c0 | (c1 << 8) | (c2 << 16) | (c3 << 24);
-        }
-        q4[0] = make_int4(words[0], words[1], words[2], words[3]);
-        q4[1] = make_int4(words[4], words[5], words[6], words[7]);
+        const int code = go_int8_code(rintf(qv / sc));
+        q8[lane] = static_cast<int8_t>(code);
         sq = sc;
     }
     __syncthreads();
 
-    // Logits: lane (key jj = lane % 32, half) dots its 32 codes; the halves
-    // add up exactly (int32), the float query sums in order on half 0.
-    for (int g = 0; g < nch; ++g) {
-        wait_chunk(g);
-        const int j0 = g * JC, cnt = min(JC, n - j0);
+    // Logits, two chunks a turn, a key per lane. A row is 64 bytes, so lanes
+    // four apart take its 16-byte pieces a piece apart: 16 lanes of a read then
+    // cover every bank. The int8 dot is exact in any order; the float query
+    // sums in order.
+    if (a.quant_q)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) q4[c] = *reinterpret_cast<const int4 *>(q8 + 16 * ((c + (lane >> 2)) & 3));
+    for (int g = 0; g < nch; g += 2) {
+        const bool two = g + 1 < nch;
+        wait_turn(g, two);
+        const int j0 = g * JC, cnt = min(2 * JC, n - j0);
         const int jj = lane & 31;
-        const int8_t *slot = ring + (g % RS) * kRingSlot;
+        const int8_t *slot = ring + ((g + (two ? lane >> 5 : 0)) % RS) * kRingSlot;
         const int8_t *row = slot + jj * ROW;
         const float kscale = reinterpret_cast<const float *>(slot + JC * ROW)[jj];
         float lg = 0.0f;
         if (a.quant_q) {
-            const int4 k0 = *reinterpret_cast<const int4 *>(row + 32 * half);
-            const int4 k1 = *reinterpret_cast<const int4 *>(row + 32 * half + 16);
             int dot = 0;
-            dot = __builtin_amdgcn_sdot4(k0.x, q4[0].x, dot, false);
-            dot = __builtin_amdgcn_sdot4(k0.y, q4[0].y, dot, false);
-            dot = __builtin_amdgcn_sdot4(k0.z, q4[0].z, dot, false);
-            dot = __builtin_amdgcn_sdot4(k0.w, q4[0].w, dot, false);
-            dot = __builtin_amdgcn_sdot4(k1.x, q4[1].x, dot, false);
-            dot = __builtin_amdgcn_sdot4(k1.y, q4[1].y, dot, false);
-            dot = __builtin_amdgcn_sdot4(k1.z, q4[1].z, dot, false);
-            dot = __builtin_amdgcn_sdot4(k1.w, q4[1].w, dot, false);
-            dot += __shfl_xor(dot, 32);
-            if (half == 0 && jj < cnt) {
-                const float scl = sq * kscale;
-                const float t1 = static_cast<float>(dot) * scl;
-                lg = t1 / a.scale;
+            int4 kw[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) kw[c] = *reinterpret_cast<const int4 *>(row + 16 * ((c + (lane >> 2)) & 3));
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                dot = __builtin_amdgcn_sdot4(kw[c].x, q4[c].x, dot, false);
+                dot = __builtin_amdgcn_sdot4(kw[c].y, q4[c].y, dot, false);
+                dot = __builtin_amdgcn_sdot4(kw[c].z, q4[c].z, dot, false);
+                dot = __builtin_amdgcn_sdot4(kw[c].w, q4[c].w, dot, false);
             }
-        } else if (half == 0 && jj < cnt) {
+            const float scl = sq * kscale;
+            const float t1 = static_cast<float>(dot) * scl;
+            lg = t1 / a.scale;
+        } else if (lane < cnt) {
             float dot = 0.0f;  // in order
             for (int c = 0; c < ROW; c += 4) {
                 const int wd = *reinterpret_cast<const int *>(row + c);
@@ -1399,8 +1405,9 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
             const float t1 = dot * kscale;
             lg = t1 / a.scale;
         }
-        if (half == 0 && jj < cnt) s[j0 + jj] = lg;
+        if (lane < cnt) s[j0 + lane] = lg;
         refill(g);
+        if (two) refill(g + 1);
     }
     __syncthreads();
 
@@ -1417,6 +1424,13 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
     if (lane < 8 && kernel_path) {  // lane k of the 8-lane sum, elements in order
         float acc = 0.0f;
         int j = lane;
+        for (; j + 120 < n8; j += 128) {
+            float e[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) e[k] = s[j + 8 * k];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) acc = acc + e[k];
+        }
         for (; j + 56 < n8; j += 64) {
             float e[8];
 #pragma unroll
@@ -1444,51 +1458,57 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
     }
     __syncthreads();
 
-    // 3. axpysI8 (int8kernel.go:360-368): the chunk's weights, then lane d's
-    // products in key order.
+    // 3. axpysI8 (int8kernel.go:360-368), two chunks a turn: their weights, a
+    // key per lane, then lane d's products in key order.
     float acc = 0.0f;
-    for (int g = nch; g < total; ++g) {
-        wait_chunk(g);
-        const int j0 = (g - nch) * JC, cnt = min(JC, n - j0);
-        const int8_t *sl = ring + (g % RS) * kRingSlot;
-        if (lane < cnt) {
+    for (int g = nch; g < total; g += 2) {
+        const bool two = g + 1 < total;
+        wait_turn(g, two);
+        const int j0 = (g - nch) * JC;
+        if (j0 + lane < min(n, j0 + 2 * JC)) {
+            const int8_t *sl = ring + ((g + (lane >> 5)) % RS) * kRingSlot;
             const float p = s[j0 + lane] / sum;
-            s[j0 + lane] = p * reinterpret_cast<const float *>(sl + JC * ROW)[lane];
+            s[j0 + lane] = p * reinterpret_cast<const float *>(sl + JC * ROW)[lane & 31];
         }
         __syncthreads();
-        const int8_t *slot = sl + lane;
-        const float *wj = s + j0;
-        if (cnt == JC) {
-            // Every code and weight read of the chunk goes out before the
-            // first product: left to itself the compiler reused 8 registers
-            // for the codes and waited on each 8 reads in turn (batch-256
-            // cross call 89.5 -> 86.8 us, bit for bit the same).
-            int ci[JC];
-            float4 wv[JC / 4];
 #pragma unroll
-            for (int k = 0; k < JC; ++k) ci[k] = slot[k * ROW];
+        for (int u = 0; u < 2; ++u) {
+            if (u == 1 && !two) break;
+            const int cnt = min(JC, n - j0 - u * JC);
+            const int8_t *slot = ring + ((g + u) % RS) * kRingSlot + lane;
+            const float *wj = s + j0 + u * JC;
+            if (cnt == JC) {
+                // Every code and weight read of the chunk goes out before the
+                // first product: left to itself the compiler reused 8 registers
+                // for the codes and waited on each 8 reads in turn (batch-256
+                // cross call 89.5 -> 86.8 us, bit for bit the same).
+                int ci[JC];
+                float4 wv[JC / 4];
 #pragma unroll
-            for (int q = 0; q < JC / 4; ++q) wv[q] = *reinterpret_cast<const float4 *>(wj + 4 * q);
-            __builtin_amdgcn_sched_barrier(0);
-            float cd[JC];
+                for (int k = 0; k < JC; ++k) ci[k] = slot[k * ROW];
 #pragma unroll
-            for (int k = 0; k < JC; ++k) cd[k] = static_cast<float>(ci[k]);
+                for (int q = 0; q < JC / 4; ++q) wv[q] = *reinterpret_cast<const float4 *>(wj + 4 * q);
+                __builtin_amdgcn_sched_barrier(0);
+                float cd[JC];
 #pragma unroll
-            for (int q = 0; q < JC / 4; ++q) {
-                const float p0 = wv[q].x * cd[4 * q], p1 = wv[q].y * cd[4 * q + 1];
-                const float p2 = wv[q].z * cd[4 * q + 2], p3 = wv[q].w * cd[4 * q + 3];
-                acc = acc + p0;
-                acc = acc + p1;
-                acc = acc + p2;
-                acc = acc + p3;
+                for (int k = 0; k < JC; ++k) cd[k] = static_cast<float>(ci[k]);
+#pragma unroll
+                for (int q = 0; q < JC / 4; ++q) {
+                    const float p0 = wv[q].x * cd[4 * q], p1 = wv[q].y * cd[4 * q + 1];
+                    const float p2 = wv[q].z * cd[4 * q + 2], p3 = wv[q].w * cd[4 * q + 3];
+                    acc = acc + p0;
+                    acc = acc + p1;
+                    acc = acc + p2;
+                    acc = acc + p3;
+                }
+            } else {
+                for (int jj = 0; jj < cnt; ++jj) {
+                    const float pr = wj[jj] * static_cast<float>(slot[jj * ROW]);
+                    acc = acc + pr;
+                }
             }
-        } else {
-            for (int jj = 0; jj < cnt; ++jj) {
-                const float pr = wj[jj] * static_cast<float>(slot[jj * ROW]);
-                acc = acc + pr;
-            }
+            refill(g + u);
         }
-        refill(g);
     }
     outp[lane] = acc;
 }
@@ -1904,12 +1924,11 @@ hipError_t launch_attend_int8(const AttendArgs &args, int cus, hipStream_t strea
             }
         }
         if (a.qk == kChainVd) {
-            // many streams: key and value chunks through a ring of 6 slots
-            // (eight workgroups per CU at 1500 keys)
-            constexpr int rs = 6;
+            // many streams: key and value chunks through a ring (ten
+            // workgroups per CU at 1500 keys)
             const size_t lds = with_pages(4 * ((static_cast<size_t>(a.nk_max) + 3) & ~size_t(3)) +
-                                          static_cast<size_t>(rs) * kRingSlot);
-            if (lds <= 150 * 1024) return launch_attend_ring<rs>(a, lds, stream);
+                                          static_cast<size_t>(kRingSlots) * kRingSlot);
+            if (lds <= 150 * 1024) return launch_attend_ring<kRingSlots>(a, lds, stream);
         }
         const int rs = 4;
         const size_t lds = with_pages(chain_lds(a, 32, rs));

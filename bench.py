@@ -213,7 +213,8 @@ def batched_gemm_leg(gw, torch, reps=5):
     Flops are the
     dense equivalent 2*M*Out*In; for the MFMA forms, mfma_util is the int8 MFMA
     work it issues (one 32x32x32 product per 64-row block, 64-activation tile,
-    position and 32x32 quadrant) over the time, against 5.0 POP/s. dense_f32
+    position and 32x32 quadrant; the 4-bit table form's residual products count
+    at their own, twofold rate) over the time, against 5.0 POP/s. dense_f32
     times the same matrix's Dense view (Exact's semantics on fp32 MFMA, the
     whole call: rotation, product and any fold); its mfma_util_fp32 is the
     fp32 MFMA work the padded 128 x 128 tiles issue over that time, against
@@ -238,8 +239,13 @@ def batched_gemm_leg(gw, torch, reps=5):
                     tile = 64 if path == "lut-mfma" else 32
                     mfmas = -(-o // 64) * 2 * (-(-M // tile) * tile // 32) * positions
                     ops = mfmas * 2 * 32 * 32 * 32
+                    peak_ops = ops
+                    if path == "lut-mfma-tab" and bits == 4:
+                        # the 4-bit split: 8 positions take one int8 product and two 32x32x64 fp6 x fp4
+                        # products of twice the work at twice the rate, instead of 8 int8 products
+                        ops, peak_ops = ops * 5 // 8, ops * 3 // 8
                     rec["mfma_TOPs"] = round(ops / us / 1e6, 1)
-                    rec["mfma_util"] = round(ops / (us * 1e-6) / INT8_PEAK_OPS, 4)
+                    rec["mfma_util"] = round(peak_ops / (us * 1e-6) / INT8_PEAK_OPS, 4)
                 # The Dense view of the same matrix: Exact's semantics on fp32
                 # MFMA (v_mfma_f32_32x32x2_f32 over 128 x 128 tiles, the
                 # activations rotated first), within float32 rounding of Exact.

@@ -1527,12 +1527,14 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
 //
 // Bound by VALU issue (1,667 instructions a pair of 448 keys, busy 61% of the
 // kernel) behind one exposed staging. Measured on MI355X, 8 heads of 64, 448
-// keys a stream, causal, against a wavefront a pair reading its own rows:
-// 4 streams x 96 rows, 2 key heads of 48 codes 31.5 -> 20.8 us (int8 values,
-// converted by each pair, 21.9); 8 key heads of 64 32.3 -> 18.3; 16 streams x
-// 32 rows 36.0 -> 23.2 (8 key heads 43.7 -> 24.0); 64 streams x 2 rows
-// 20.8 -> 18.0. Loading a thread's whole share before its first store, the
-// query's with it: 21.5 (92 registers for 60).
+// keys a stream, causal, against a wavefront a pair reading its own rows (the
+// chain kernel at 48 codes a key head, the ring at 64): 4 streams x 96 rows, 2
+// key heads of 48 codes 31.3 -> 20.8 us (int8 values, converted by each pair,
+// 21.9); 8 key heads of 64 22.4 -> 18.5; 16 streams x 32 rows 36.2 -> 23.2 (8
+// key heads of 64 35.1 -> 24.0); 64 streams x 2 rows 20.5 -> 18.0; the closest,
+// 64 streams x 8 rows of 8 key heads of 64, 35.3 against 35.9. Loading a thread's
+// whole share before its first store, the query's with it: 21.5 (92 registers
+// for 60).
 constexpr int kRowsMaxWaves = 16;
 
 using half2v = __attribute__((ext_vector_type(2))) _Float16;
@@ -1905,7 +1907,7 @@ hipError_t launch_attend_int8(const AttendArgs &args, int cus, hipStream_t strea
         // Prompts of more workgroups than stay resident: a workgroup of 4 to 16
         // pairs, about one for each CU. Fewer than eight wavefronts need a CU
         // each, or LDS for two workgroups on one: 128 streams x 4 rows of 8
-        // key heads took 65 us with four alone on a CU, 49.6 the way below.
+        // key heads took 65 us with four alone on a CU, 39 the way below.
         if (a.t > 1) {
             const int kv_heads = a.k_cols / a.qk, pairs = a.t * (a.heads / kv_heads);
             const long long groups = static_cast<long long>(a.batch) * kv_heads, total = groups * pairs;

@@ -1433,6 +1433,12 @@ int cq_gemms_append_dev(int n, cq_matrix *const *ms, float *const *dsts, const f
     return run_lut(ms, n, dsts, x, rows, static_cast<hipStream_t>(stream), &f);
 }
 
+// A tile's 4-bit and 2-bit tables take the same bytes, so a buffer of 4-bit
+// tables is kTabWidth4 bytes longer: a consumer knows a buffer by its size, and
+// one built for the other width is refused (a width's own sizes are 65,664
+// bytes a tile and group apart).
+constexpr size_t kTabWidth4 = 256;
+
 size_t cq_tables_bytes(int n, cq_matrix *const *ms, int rows) {
     if (n <= 0 || n > kKernargJobs || !ms || rows <= 0) return 0;
     for (int k = 0; k < n; ++k)
@@ -1440,7 +1446,7 @@ size_t cq_tables_bytes(int n, cq_matrix *const *ms, int rows) {
     if (!tab_pays(ms, n, rows)) return 0;
     const CqStore &s0 = *ms[0]->st;
     const int tiles = (rows + 31) / 32;
-    return tab_table_bytes(s0.groups, tiles) + tab_step_bytes(s0.groups, tiles);
+    return tab_table_bytes(s0.groups, tiles) + tab_step_bytes(s0.groups, tiles) + (s0.width == 4 ? kTabWidth4 : 0);
 }
 
 int cq_gemm_tables_dev(const cq_matrix *m, float *dst, const float *x, const float *gate, int rows, const float *resid,

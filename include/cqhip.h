@@ -203,7 +203,7 @@ int cq_gemm_tables_dev(const cq_matrix *m, float *dst, const float *x, const flo
  * cq_gemms_fused_dev (resid, act) and cq_gemms_append_dev (kv_q null: no
  * appends). The norm and the input are those the tables were built from.
  * CQ_ERR_MISUSE where cq_tables_bytes(n, ms, rows) is 0 or differs from
- * tables_bytes. */
+ * tables_bytes (tables of the other index width always differ). */
 int cq_gemms_tables_dev(int n, cq_matrix *const *ms, float *const *dsts, int rows, const float *resid, int act,
                         int8_t *const *kv_q, float *const *kv_s, long long q_stride, long long s_stride,
                         const int32_t *pos, int cap, const float *const *cos_t, const float *const *sin_t,

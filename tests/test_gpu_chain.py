@@ -185,6 +185,26 @@ def test_chain_unbuilt_and_misuse():
         cq.gemm_tables_dev(cq.New(p2), y2, _t(x2), 256, head, buf, resid=y2)  # the wrong size
 
 
+@pytest.mark.parametrize("built_bits,used_bits", [(2, 4), (4, 2)])
+def test_chain_refuses_tables_of_the_other_width(built_bits, used_bits):
+    # a consumer knows a table buffer by its size, so a product of the same
+    # inputs and rows at the other index width needs another size
+    import torch
+
+    D, rows = 512, 256
+    g = synth.rng(7300 + built_bits)
+    p, x, _, resid, _ = _produce(g, "down", rows)
+    nxt = {b: [cq.New(synth.random_packed(g, 2048, D, 128, b, sigma=0.05))] for b in (2, 4)}
+    gain = np.ones(D, np.float32)
+    _, tables, built = _chain(cq.New(p), x, None, resid, rows, nxt[built_bits], gain)
+    assert built and tables.numel() == cq.tables_bytes(nxt[built_bits], rows)
+    out = torch.full((rows, 2048), 7.0, device="cuda")
+    with pytest.raises(CQPanic):
+        cq.gemms_tables_dev(nxt[used_bits], [out], rows, tables)
+    torch.cuda.synchronize()
+    assert bool((out == 7.0).all())
+
+
 def test_decoder_chained_equals_unchained():
     # the synthetic decoder at 256 streams: wo, cross-wo and FFN-down build
     # the next products' tables (cross q/gate, FFN up, the next q/k/v/gate

@@ -237,6 +237,9 @@ size_t lut_tout_lds_bytes(int in);
 hipError_t launch_lut(const LutLaunch &a, int bits, int group_bytes, int waves, int grid_x, int grid_y, size_t lds,
                       hipStream_t stream);
 bool lut_geometry_supported(int bits, int group_bytes);
+// Workgroups of `threads` threads that one launch takes along x: HIP refuses a
+// grid of 2^32 work-items or more.
+inline long long grid_limit(int threads) { return 0xffffffffLL / threads; }
 // The lut product of few rows (lut_few_kernel; no prologue or epilogue): out
 // rows over all jobs, groups * ceil(out / 32) at most 16.
 hipError_t launch_lut_few(const LutLaunch &a, int bits, int out, hipStream_t s);

@@ -36,6 +36,7 @@
 
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <cstddef>
 
 namespace cqhip {
@@ -1223,14 +1224,23 @@ hipError_t launch_lut_few(const LutLaunch &a, int bits, int out, hipStream_t s) 
     const int rows = a.jobs[0].rows, groups = a.jobs[0].groups;
     const long long waves = static_cast<long long>(groups) * ((out + 31) / 32);
     if (a.njobs <= 0 || rows <= 0 || out <= 0 || groups <= 0 || waves > 16) return hipErrorInvalidValue;
-    const dim3 grid(rows), block(64 * static_cast<unsigned>(waves));
-    if (bits == 4)
-        hipLaunchKernelGGL((lut_few_kernel<4>), grid, block, 0, s, a);
-    else if (bits == 2)
-        hipLaunchKernelGGL((lut_few_kernel<2>), grid, block, 0, s, a);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
+    if (bits != 4 && bits != 2) return hipErrorInvalidValue;
+    const dim3 block(64 * static_cast<unsigned>(waves));
+    const long long most = grid_limit(block.x);  // activations of one launch
+    for (long long r0 = 0; r0 < rows; r0 += most) {
+        LutLaunch b = a;
+        for (int k = 0; k < a.njobs; ++k) {
+            b.jobs[k].x = a.jobs[k].x + r0 * a.jobs[k].x_stride;
+            b.jobs[k].y = a.jobs[k].y + r0 * a.jobs[k].y_stride;
+        }
+        const dim3 grid(static_cast<unsigned>(std::min(most, rows - r0)));
+        if (bits == 4)
+            hipLaunchKernelGGL((lut_few_kernel<4>), grid, block, 0, s, b);
+        else
+            hipLaunchKernelGGL((lut_few_kernel<2>), grid, block, 0, s, b);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 size_t lut_lds_bytes(int bits, int group_bytes, int gc, int tb, int bpw) {

@@ -1,0 +1,44 @@
+"""Calls of more work than one launch's grid can hold (HIP refuses 2^32
+work-items): their launches are split. Each call repeats a period of rows, and
+every period's result is the first one's, bit for bit the oracle's."""
+
+import numpy as np
+import pytest
+
+from go_whistle_amd import cq, synth
+from oracle import binding as orc
+
+pytestmark = pytest.mark.gpu
+
+PERIOD = 1024
+
+
+def _repeat(base, n):
+    """n rows of base, over and over, on the device."""
+    import torch
+
+    return torch.from_numpy(base).cuda().repeat(-(-n // len(base)), *[1] * (base.ndim - 1))[:n].contiguous()
+
+
+def _same(got, base):
+    """Every row of got is base's row at its place in the period."""
+    import torch
+
+    whole = len(got) // len(base)
+    want, bits = torch.from_numpy(np.ascontiguousarray(base)).cuda(), {4: torch.int32, 1: torch.int8}[got.element_size()]
+    want, got = want.view(bits), got.view(bits)
+    return bool((got[:whole * len(base)].view(whole, *want.shape) == want).all()) and \
+        torch.equal(got[whole * len(base):], want[:len(got) - whole * len(base)])
+
+
+def test_few_rows_product():
+    # one matrix row over one group: a wavefront an activation
+    import torch
+
+    rows = (1 << 26) + 5
+    g = synth.rng(4)
+    p = synth.random_packed(g, 1, 4, 128, 4, sigma=0.05)
+    x = g.standard_normal((PERIOD, 4)).astype(np.float32)
+    y = torch.full((rows, 1), 7.0, device="cuda")
+    cq.gemms_dev([cq.New(p)], [y], _repeat(x, rows), rows)
+    assert _same(y, orc.OMatrix.new(p).gemm(x.reshape(-1), PERIOD, orc.LUT).reshape(PERIOD, 1))

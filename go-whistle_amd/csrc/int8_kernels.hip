@@ -119,8 +119,9 @@ constexpr int kQuantVecMax = 2048;  // values of a chunk the kernel holds in reg
 template <bool FAKE>
 hipError_t launch_quant_vec(int8_t *q, float *s, float *dst, const float *x, long long chunks, int width, hipStream_t stream) {
     const int per = width <= 64 ? 16 : 4;  // chunks a workgroup
-    for (long long c0 = 0; c0 < chunks; c0 += static_cast<long long>(per) << 24) {
-        const long long n = std::min(chunks - c0, static_cast<long long>(per) << 24);
+    const long long most = per * grid_limit(256);
+    for (long long c0 = 0; c0 < chunks; c0 += most) {
+        const long long n = std::min(chunks - c0, most);
         const dim3 grid(static_cast<unsigned>((n + per - 1) / per));
         int8_t *qc = FAKE ? nullptr : q + c0 * width;
         float *scl = FAKE ? nullptr : s + c0, *dc = FAKE ? dst + c0 * width : nullptr;
@@ -1790,9 +1791,9 @@ hipError_t launch_fake_quant(float *dst, const float *x, long long chunks, int w
     if ((width & 3) == 0 && width <= kQuantVecMax &&
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0)
         return launch_quant_vec<true>(nullptr, nullptr, dst, x, chunks, width, stream);
-    const long long blocks = (chunks + 3) / 4;
-    for (long long c0 = 0; c0 < blocks; c0 += 1 << 30) {
-        const long long nb = blocks - c0 < (1LL << 30) ? blocks - c0 : (1LL << 30);
+    const long long blocks = (chunks + 3) / 4, most = grid_limit(256);
+    for (long long c0 = 0; c0 < blocks; c0 += most) {
+        const long long nb = std::min(blocks - c0, most);
         const long long ch0 = c0 * 4;
         hipLaunchKernelGGL(fake_quant_kernel, dim3(static_cast<unsigned>(nb)), dim3(256), 0, stream, dst + ch0 * width,
                            x + ch0 * width, chunks - ch0, width);
@@ -1808,9 +1809,9 @@ hipError_t launch_quantize_rows(int8_t *q, float *s, const float *x, long long c
     if ((width & 3) == 0 && width <= kQuantVecMax && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
         (reinterpret_cast<uintptr_t>(q) & 3) == 0)
         return launch_quant_vec<false>(q, s, nullptr, x, chunks, width, stream);
-    const long long blocks = (chunks + 3) / 4;
-    for (long long c0 = 0; c0 < blocks; c0 += 1 << 30) {
-        const long long nb = blocks - c0 < (1LL << 30) ? blocks - c0 : (1LL << 30);
+    const long long blocks = (chunks + 3) / 4, most = grid_limit(256);
+    for (long long c0 = 0; c0 < blocks; c0 += most) {
+        const long long nb = std::min(blocks - c0, most);
         const long long ch0 = c0 * 4;
         hipLaunchKernelGGL(quantize_kernel, dim3(static_cast<unsigned>(nb)), dim3(256), 0, stream, q + ch0 * width,
                            s + ch0, x + ch0 * width, chunks - ch0, width);

@@ -5,7 +5,7 @@ every period's result is the first one's, bit for bit the oracle's."""
 import numpy as np
 import pytest
 
-from go_whistle_amd import cq, synth
+from go_whistle_amd import cq, needle, synth
 from oracle import binding as orc
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +42,19 @@ def test_few_rows_product():
     y = torch.full((rows, 1), 7.0, device="cuda")
     cq.gemms_dev([cq.New(p)], [y], _repeat(x, rows), rows)
     assert _same(y, orc.OMatrix.new(p).gemm(x.reshape(-1), PERIOD, orc.LUT).reshape(PERIOD, 1))
+
+
+@pytest.mark.parametrize("width,chunks", [(4, (1 << 28) + 5), (1, (1 << 26) + 5)])  # float4s, 16 lanes a chunk; the rest, 64
+def test_quantise_rows_and_fake_quant(width, chunks):
+    import torch
+
+    x = (np.random.default_rng(width).standard_normal((PERIOD, width)) ** 3).astype(np.float32)
+    q, s = orc.quantize_rows(x.reshape(-1), width, width)
+    xd = _repeat(x, chunks)
+    qd, sd = torch.full((chunks, width), 99, dtype=torch.int8, device="cuda"), torch.full((chunks,), 9.0, device="cuda")
+    needle.quantize_rows_dev(qd, sd, xd, chunks, width, width)
+    assert _same(qd, q.reshape(PERIOD, width)) and _same(sd, s)
+    del qd, sd
+    needle.fake_quant_dev(xd, xd, chunks, width, width)
+    want = q.reshape(PERIOD, width).astype(np.float32) * s[:, None]
+    assert _same(xd, want.astype(np.float32))

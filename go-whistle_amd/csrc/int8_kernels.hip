@@ -1918,7 +1918,7 @@ hipError_t launch_attend_int8(const AttendArgs &args, int cus, hipStream_t strea
             const int per_group = (pairs + nw - 1) / nw;
             const size_t lds = with_pages(rows_lds(a, nw));
             const bool enough = nw >= 8 || groups * per_group <= cus || 2 * lds <= 150 * 1024;
-            if (nw >= 4 && enough && lds <= 150 * 1024 && groups * per_group <= INT_MAX) {
+            if (nw >= 4 && enough && lds <= 150 * 1024 && groups * per_group <= grid_limit(64 * nw)) {
                 static std::atomic<unsigned long long> attr{0};
                 if (hipError_t e = lds_limit_once(reinterpret_cast<const void *>(&attend_rows_kernel), 152 * 1024, attr)) return e;
                 hipLaunchKernelGGL(attend_rows_kernel, dim3(static_cast<unsigned>(groups * per_group)), dim3(64 * nw), lds, stream,

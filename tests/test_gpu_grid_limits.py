@@ -58,3 +58,23 @@ def test_quantise_rows_and_fake_quant(width, chunks):
     needle.fake_quant_dev(xd, xd, chunks, width, width)
     want = q.reshape(PERIOD, width).astype(np.float32) * s[:, None]
     assert _same(xd, want.astype(np.float32))
+
+
+def test_prompt_attention():
+    # 17 pairs a stream in workgroups of 16 wavefronts: two a stream, the
+    # second nearly empty, 2^32 threads where a wavefront a pair has 2^31
+    import torch
+
+    batch, t, qk, vd, nk = 1 << 21, 17, 16, 64, 4
+    g = np.random.default_rng(17)
+    kq, vq = (g.integers(-128, 128, (nk, w), dtype=np.int8) for w in (qk, vd))
+    ks, vs = ((g.random((nk, 1)) * 0.05 + 1e-3).astype(np.float32) for _ in range(2))
+    q = g.standard_normal((PERIOD, t * qk)).astype(np.float32)
+    spans = np.tile(np.array([[0, 0, 0, nk]], np.int32), (PERIOD * t, 1))
+    out = torch.full((batch, t * vd), 7.0, device="cuda")
+    dev = lambda a: torch.from_numpy(a).cuda()
+    needle.attend_int8_dev(out, _repeat(q, batch), t, 1, dev(kq), dev(ks), qk, qk, dev(vq), dev(vs), vd, vd,
+                           _repeat(spans, batch * t), nk, 4.0, True, batch=batch, kv_stride=0, s_stride=0)
+    want = orc.attend_int8_spans(q.reshape(-1), PERIOD * t, 1, kq.reshape(-1), ks.reshape(-1), qk, qk, vq.reshape(-1),
+                                 vs.reshape(-1), vd, vd, nk, spans, np.float32(4.0), True, 1)
+    assert _same(out, want.reshape(PERIOD, t * vd))

@@ -2151,7 +2151,7 @@ int nd_hadamard_mlp_dev(float *out, const float *x, int rows, int dim, int na, i
 
 int nd_rms_unit_dev(float *dst, const float *x, int rows, int dim, void *stream) {
     if (rows < 0 || dim <= 0) return fail(CQ_ERR_MISUSE, "needle: RMSUnit of %d rows of %d", rows, dim);
-    if (row_unit_dim(dim))  // 256 threads a row, the squares' chains read ahead from LDS
+    if (row_unit_pays(rows, dim))  // 256 threads a row, the squares' chains read ahead from LDS
         HIP_TRY(launch_rms_unit_row(dst, x, rows, dim, 0, static_cast<hipStream_t>(stream)), "RMSUnit launch");
     else
         HIP_TRY(launch_rms_unit(dst, x, rows, dim, static_cast<hipStream_t>(stream)), "RMSUnit launch");

@@ -458,7 +458,7 @@ hipError_t launch_qkv_prep(const PrepArgs &a, int batch, hipStream_t s);
 // resid + float32(sc * ZCRMSNorm(y)); RMSUnit, with quant then fakeQuant of
 // the whole row.
 bool row_kernel_dim(int dim);
-bool row_unit_dim(int dim);  // rows launch_rms_unit_row takes without quant
+bool row_unit_pays(int rows, int dim);  // rows that launch_rms_unit_row takes without quant, and faster than launch_rms_unit
 hipError_t launch_norm_scaled_add(float *h, const float *resid, const float *y, const float *gain, float sc, int rows,
                                   int dim, hipStream_t s);
 hipError_t launch_rms_unit_row(float *dst, const float *x, int rows, int dim, int quant, hipStream_t s);

@@ -21,6 +21,8 @@
 #include "cq_internal.hpp"
 #include "cq_device.hpp"
 
+#include <type_traits>
+
 namespace cqhip {
 namespace {
 
@@ -98,11 +100,12 @@ __global__ __launch_bounds__(1024) void qkv_prep_kernel(PrepArgs a) {
 // partial, [i mod 4][i / 4], and lanes 0-3 of wavefront 0 only add them, in
 // order, 16 reads ahead of the adds; a tail of dim mod 4 values follows in
 // partial 0 (norm.go:91-109). Returns the sum of squares to every thread.
-// The chain of dim / 4 dependent float64 adds bounds these kernels. With the
-// converts and squares in the chain as well (float squares staged, each lane
-// converting and squaring its values between the adds) RMSUnit of 2048 took
-// 7.2 us a launch of one row and 10.7 us for 375 rows, against 4.9 and 8.8 us
-// (MI355X, kernel trace).
+// The chain of dim / 4 dependent float64 adds bounds these kernels at few rows;
+// at many, the float64 squares' LDS traffic and the waves' turnover. Measured on
+// MI355X (us a call from a graph, RMSUnit of 2048 at 1, 375 and 12,000 rows):
+// 6.2, 8.2, 64.0, against 7.7, 10.8, 79.5 with the converts and squares in the
+// chain (float squares staged, each lane converting and squaring its values
+// between the adds).
 constexpr int kRowMax = 4096;
 
 // Doubles from one partial's squares to the next: 16-byte reads of the four
@@ -110,14 +113,14 @@ constexpr int kRowMax = 4096;
 __host__ __device__ constexpr int row_stride(int dim) { return ((dim >> 2) + 31) / 32 * 32 + 2; }
 size_t row_lds(int dim) { return (4 * static_cast<size_t>(row_stride(dim)) + 4) * sizeof(double); }
 
-__device__ __forceinline__ double row_square_sum(const float *row, int dim, float (&v)[kRowMax / 256], double *t,
-                                                 double *sum_sh) {
+template <int V>
+__device__ __forceinline__ double row_square_sum(const float *row, int dim, float (&v)[V], double *t, double *sum_sh) {
     const int tid = threadIdx.x;
     const int q = dim >> 2, full = dim & ~3, stride = row_stride(dim);
 #pragma unroll
-    for (int e = 0; e < kRowMax / 256; ++e) v[e] = tid + 256 * e < dim ? row[tid + 256 * e] : 0.0f;
+    for (int e = 0; e < V; ++e) v[e] = tid + 256 * e < dim ? row[tid + 256 * e] : 0.0f;
 #pragma unroll
-    for (int e = 0; e < kRowMax / 256; ++e) {
+    for (int e = 0; e < V; ++e) {
         const int i = tid + 256 * e;
         const double d = v[e];
         if (i < dim) t[i < full ? (i & 3) * stride + (i >> 2) : 4 * stride + (i - full)] = d * d;
@@ -161,12 +164,13 @@ __device__ __forceinline__ double row_square_sum(const float *row, int dim, floa
 }
 
 // h = resid + float32(s * ZCRMSNorm(y)) per row (resid may be h).
+template <int V>
 __global__ __launch_bounds__(256) void norm_scaled_add_kernel(float *h, const float *resid, const float *y,
                                                               const float *gain, float s, int dim) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double sum_sh;
     const int r = blockIdx.x, tid = threadIdx.x;
-    float v[kRowMax / 256];
+    float v[V];
     const double sum = row_square_sum(y + static_cast<long long>(r) * dim, dim, v, reinterpret_cast<double *>(smem), &sum_sh);
     // zc_rms: float32(sqrt(float64(float32(s / dim) + 1e-6)))
     const float ms = static_cast<float>(sum / static_cast<double>(dim));
@@ -175,7 +179,7 @@ __global__ __launch_bounds__(256) void norm_scaled_add_kernel(float *h, const fl
     const float *rr = resid + static_cast<long long>(r) * dim;
     float *hr = h + static_cast<long long>(r) * dim;
 #pragma unroll
-    for (int k = 0; k < kRowMax / 256; ++k)
+    for (int k = 0; k < V; ++k)
         if (k < (dim >> 8)) {
             const int c = tid + 256 * k;
             const float gx = gain[c] * v[k];
@@ -189,22 +193,23 @@ __global__ __launch_bounds__(256) void norm_scaled_add_kernel(float *h, const fl
 // 1e-6))); with quant, then the fakeQuant of the whole row (int8.go:57-75,
 // one chunk of dim): the mHC phi products' int8 input (mhc.go:99-106,
 // linear.go:80-87).
+template <int V>
 __global__ __launch_bounds__(256) void rms_unit_row_kernel(float *dst, const float *x, int dim, int quant) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double sum_sh;
     __shared__ float red[4];
     const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float v[kRowMax / 256];
+    float v[V];
     const double sum = row_square_sum(x + static_cast<long long>(r) * dim, dim, v, reinterpret_cast<double *>(smem), &sum_sh);
     const float ms = static_cast<float>(sum / static_cast<double>(dim));
     const float e = ms + 1e-6f;
     const float inv = static_cast<float>(1.0 / sqrt(static_cast<double>(e)));
 #pragma unroll
-    for (int k = 0; k < kRowMax / 256; ++k) v[k] = v[k] * inv;
+    for (int k = 0; k < V; ++k) v[k] = v[k] * inv;
     if (quant) {  // QuantizeRow's bound with Go's NaN-keeping max, then code * scale
         float m = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kRowMax / 256; ++k)
+        for (int k = 0; k < V; ++k)
             if (tid + 256 * k < dim) m = go_max(m, fabsf(v[k]));
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) m = go_max(m, __shfl_xor(m, off));
@@ -213,12 +218,12 @@ __global__ __launch_bounds__(256) void rms_unit_row_kernel(float *dst, const flo
         m = go_max(go_max(red[0], red[1]), go_max(red[2], red[3]));
         const float sc = m > 0.0f ? m / 127.0f : 1.0f;
 #pragma unroll
-        for (int k = 0; k < kRowMax / 256; ++k)
+        for (int k = 0; k < V; ++k)
             if (tid + 256 * k < dim) v[k] = static_cast<float>(go_int8_code(rintf(v[k] / sc))) * sc;
     }
     float *out = dst + static_cast<long long>(r) * dim;
 #pragma unroll
-    for (int k = 0; k < kRowMax / 256; ++k)
+    for (int k = 0; k < V; ++k)
         if (tid + 256 * k < dim) out[tid + 256 * k] = v[k];
 }
 
@@ -282,19 +287,51 @@ hipError_t launch_qkv_prep(const PrepArgs &a, int batch, hipStream_t s) {
 }
 
 bool row_kernel_dim(int dim) { return dim > 0 && dim % 256 == 0 && dim <= kRowMax; }
-bool row_unit_dim(int dim) { return dim > 0 && dim <= kRowMax; }
+
+// Rows that RMSUnit runs on 256 threads a row; the others on a wavefront a row
+// (rms_unit_kernel), which wins where rows fill the chip and are so narrow that
+// most of 256 threads have nothing to do. Measured on MI355X (us, 256 threads
+// against a wavefront): rows of 64 at 375, 1000, 3000 and 12,000 rows 2.5, 2.9,
+// 4.3, 10.5 against 2.6, 2.8, 3.4, 6.2; of 128 at 1500, 2000 and 3000 3.4, 3.9,
+// 4.7 against 3.9, 4.0, 4.2; of 256 at 3000, 6000 and 12,000 5.7, 8.9, 15.2
+// against 5.8, 8.2, 12.6; of 384 at 3000 and 12,000 6.7, 18.4 against 7.4, 21.1.
+constexpr int kNarrowRow = 256;
+bool row_unit_pays(int rows, int dim) {
+    return dim > 0 && dim <= kRowMax && (dim > kNarrowRow || rows <= 16LL * dim);
+}
+
+namespace {
+// A thread's values of a row, V: the least power of two that covers it. A load
+// or store masked off past the row costs nearly a real one: with V = 16 at every
+// width, RMSUnit of 256, 512 and 2048 took 27.7, 34.6 and 75.9 us at 12,000 rows,
+// 15.2, 21.7 and 64.0 so; uniform branches around them instead split the loads
+// of a wide row (2048 at one row 6.9 us, 6.2 so).
+template <class F>
+hipError_t by_row_values(int dim, F launch) {
+    if (dim <= 256) return launch(std::integral_constant<int, 1>{});
+    if (dim <= 512) return launch(std::integral_constant<int, 2>{});
+    if (dim <= 1024) return launch(std::integral_constant<int, 4>{});
+    if (dim <= 2048) return launch(std::integral_constant<int, 8>{});
+    return launch(std::integral_constant<int, kRowMax / 256>{});
+}
+}  // namespace
 
 hipError_t launch_norm_scaled_add(float *h, const float *resid, const float *y, const float *gain, float sc, int rows,
                                   int dim, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(norm_scaled_add_kernel, dim3(rows), dim3(256), row_lds(dim), s, h, resid, y, gain, sc, dim);
-    return hipGetLastError();
+    return by_row_values(dim, [&](auto v) {
+        hipLaunchKernelGGL((norm_scaled_add_kernel<decltype(v)::value>), dim3(rows), dim3(256), row_lds(dim), s, h, resid, y,
+                           gain, sc, dim);
+        return hipGetLastError();
+    });
 }
 
 hipError_t launch_rms_unit_row(float *dst, const float *x, int rows, int dim, int quant, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(rms_unit_row_kernel, dim3(rows), dim3(256), row_lds(dim), s, dst, x, dim, quant);
-    return hipGetLastError();
+    return by_row_values(dim, [&](auto v) {
+        hipLaunchKernelGGL((rms_unit_row_kernel<decltype(v)::value>), dim3(rows), dim3(256), row_lds(dim), s, dst, x, dim, quant);
+        return hipGetLastError();
+    });
 }
 
 hipError_t launch_expand_lanes(float *stream, const float *x, int rows, int lanes, int dim, hipStream_t s) {

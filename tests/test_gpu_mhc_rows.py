@@ -36,6 +36,20 @@ def test_rms_unit_widths(dim):
     assert same(y.cpu().numpy(), orc.rms_unit(x, rows, dim))
 
 
+@pytest.mark.parametrize("dim,rows", [(1, 16), (1, 17), (5, 80), (5, 81), (64, 1024), (64, 1025), (255, 4081), (256, 4096),
+                                      (256, 4097), (257, 4200), (512, 9), (1025, 5), (2049, 5)])
+def test_rms_unit_row_counts(dim, rows):
+    # either side of the rows that a wavefront a row takes, and of the widths
+    # at which a thread's values double
+    import torch
+
+    x = (np.random.default_rng(dim + rows).standard_normal((rows, dim)) * 3).astype(np.float32)
+    y = torch.full((rows, dim), 9.0, device="cuda")
+    needle.rms_unit_dev(y, _t(x), rows, dim)
+    torch.cuda.synchronize()
+    assert same(y.cpu().numpy(), orc.rms_unit(x, rows, dim))
+
+
 @pytest.mark.parametrize("lanes", [1, 2, 3, 4, 8])
 @pytest.mark.parametrize("dim,offset", [(512, 0), (512, 1), (1540, 0), (5, 0), (70, 0), (4, 0)])
 def test_heads_and_mix(lanes, dim, offset):

@@ -21,6 +21,7 @@
 #include "cq_internal.hpp"
 #include "cq_device.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace cqhip {
@@ -327,11 +328,17 @@ hipError_t launch_norm_scaled_add(float *h, const float *resid, const float *y, 
 }
 
 hipError_t launch_rms_unit_row(float *dst, const float *x, int rows, int dim, int quant, hipStream_t s) {
-    if (rows <= 0) return hipSuccess;
-    return by_row_values(dim, [&](auto v) {
-        hipLaunchKernelGGL((rms_unit_row_kernel<decltype(v)::value>), dim3(rows), dim3(256), row_lds(dim), s, dst, x, dim, quant);
-        return hipGetLastError();
-    });
+    const long long most = grid_limit(256);
+    for (long long r0 = 0; r0 < rows; r0 += most) {
+        const dim3 grid(static_cast<unsigned>(std::min(most, rows - r0)));
+        const hipError_t e = by_row_values(dim, [&](auto v) {
+            hipLaunchKernelGGL((rms_unit_row_kernel<decltype(v)::value>), grid, dim3(256), row_lds(dim), s, dst + r0 * dim,
+                               x + r0 * dim, dim, quant);
+            return hipGetLastError();
+        });
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_expand_lanes(float *stream, const float *x, int rows, int lanes, int dim, hipStream_t s) {

@@ -11,6 +11,8 @@
 #include "cq_internal.hpp"
 #include "cq_device.hpp"
 
+#include <algorithm>
+
 namespace cqhip {
 namespace {
 
@@ -277,9 +279,13 @@ __global__ __launch_bounds__(256) void mhc_mix_kernel(MhcArgs m) {
 bool mhc_shape_ok(int lanes, int dim) { return lanes > 0 && lanes <= kMhcMaxLanes && dim > 0; }
 
 hipError_t launch_rms_unit(float *dst, const float *x, int rows, int dim, hipStream_t s) {
-    if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(rms_unit_kernel, dim3(static_cast<unsigned>(rows)), dim3(64), 0, s, dst, x, dim);
-    return hipGetLastError();
+    const long long most = grid_limit(64);
+    for (long long r0 = 0; r0 < rows; r0 += most) {
+        const dim3 grid(static_cast<unsigned>(std::min(most, rows - r0)));
+        hipLaunchKernelGGL(rms_unit_kernel, grid, dim3(64), 0, s, dst + r0 * dim, x + r0 * dim, dim);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_mhc_heads(const MhcArgs &m, int rows, hipStream_t s) {

@@ -78,3 +78,13 @@ def test_prompt_attention():
     want = orc.attend_int8_spans(q.reshape(-1), PERIOD * t, 1, kq.reshape(-1), ks.reshape(-1), qk, qk, vq.reshape(-1),
                                  vs.reshape(-1), vd, vd, nk, spans, np.float32(4.0), True, 1)
     assert _same(out, want.reshape(PERIOD, t * vd))
+
+
+def test_rms_unit():
+    import torch
+
+    rows = (1 << 26) + 5
+    x = np.random.default_rng(8).standard_normal((PERIOD, 1)).astype(np.float32)
+    y = torch.full((rows, 1), 9.0, device="cuda")
+    needle.rms_unit_dev(y, _repeat(x, rows), rows, 1)
+    assert _same(y, orc.rms_unit(x, PERIOD, 1).reshape(PERIOD, 1))

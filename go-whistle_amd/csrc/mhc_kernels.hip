@@ -214,52 +214,70 @@ __global__ __launch_bounds__(256) void mhc_heads_kernel(MhcArgs m) {
     }
 }
 
-// The lane mix, a workgroup per row: a thread reads its columns of every
-// lane once for all the output lanes (a workgroup per output lane read the
-// stream n times: one row of 4 x 512 2.4 -> 1.5 us, 375 rows 5.3 -> 4.8 us,
-// mostly the launch's latency).
-template <int V>
-__global__ __launch_bounds__(256) void mhc_mix_kernel(MhcArgs m) {
-    const int i = blockIdx.x, n = m.lanes, dim = m.dim;
+// The lane mix, a workgroup per row and `per` output lanes (ONE: one): a thread
+// reads its columns of every lane once for them. The coefficients come in beside
+// the stream's values, into registers for one output lane and into LDS for the
+// loop over several, where reading them from memory lane by lane cost a load's
+// latency each.
+template <int V, bool ONE>
+__global__ __launch_bounds__(256) void mhc_mix_kernel(MhcArgs m, int per) {
+    __shared__ float hs[ONE ? 1 : kMhcMaxLanes * kMhcMaxLanes], qs[kMhcMaxLanes];
+    const int i = blockIdx.x, n = m.lanes, dim = m.dim, tid = threadIdx.x;
+    const int a0 = blockIdx.y * per, cnt = ONE ? 1 : min(per, n - a0);
     const float *st = m.stream + static_cast<long long>(i) * n * dim;
-    const float *hr = m.h_res + static_cast<long long>(i) * n * n, *hq = m.h_post + static_cast<long long>(i) * n;
     const float *bo = m.block_out + static_cast<long long>(i) * dim, *uo = m.u + static_cast<long long>(i) * dim;
-    float *o = m.out + static_cast<long long>(i) * n * dim;
-    for (int c = threadIdx.x * V; c < dim; c += blockDim.x * V) {
-        float sv[kMhcMaxLanes][V], y[V], bv[V], uv[V];
-        auto load = [&](float (&d)[V], const float *p) {
-            if constexpr (V == 4) {
-                const float4 f = *reinterpret_cast<const float4 *>(p);
-                d[0] = f.x;
-                d[1] = f.y;
-                d[2] = f.z;
-                d[3] = f.w;
-            } else {
-                d[0] = *p;
-            }
-        };
+    const float *hr = m.h_res + (static_cast<long long>(i) * n + a0) * n, *hq = m.h_post + static_cast<long long>(i) * n + a0;
+    float *o = m.out + (static_cast<long long>(i) * n + a0) * dim;
+    float sv[kMhcMaxLanes][V], bv[V], uv[V];
+    auto load = [&](float (&d)[V], const float *p) {
+        if constexpr (V == 4) {
+            const float4 f = *reinterpret_cast<const float4 *>(p);
+            d[0] = f.x;
+            d[1] = f.y;
+            d[2] = f.z;
+            d[3] = f.w;
+        } else {
+            d[0] = *p;
+        }
+    };
+    auto columns = [&](int c) {
         load(bv, bo + c);
         load(uv, uo + c);
 #pragma unroll
         for (int b = 0; b < kMhcMaxLanes; ++b)
             if (b < n) load(sv[b], st + static_cast<long long>(b) * dim + c);
+    };
+    int c = tid * V;
+    if (c < dim) columns(c);
+    float h1[kMhcMaxLanes], q1 = 0.0f;
+    if constexpr (ONE) {
+#pragma unroll
+        for (int b = 0; b < kMhcMaxLanes; ++b) h1[b] = b < n ? hr[b] : 0.0f;
+        q1 = hq[0];
+    } else {
+        if (tid < cnt * n) hs[tid] = hr[tid];
+        if (tid < cnt) qs[tid] = hq[tid];
+        __syncthreads();
+    }
+    while (c < dim) {
+        float y[V];
 #pragma unroll
         for (int q = 0; q < V; ++q) y[q] = bv[q] - uv[q];
-        for (int a = 0; a < n; ++a) {
+        for (int a = 0; a < cnt; ++a) {
             float v[V];
 #pragma unroll
             for (int q = 0; q < V; ++q) v[q] = 0.0f;
 #pragma unroll
             for (int b = 0; b < kMhcMaxLanes; ++b)
                 if (b < n) {
-                    const float h = hr[a * n + b];
+                    const float h = ONE ? h1[b] : hs[a * n + b];
 #pragma unroll
                     for (int q = 0; q < V; ++q) {
                         const float pr = h * sv[b][q];
                         v[q] = v[q] + pr;
                     }
                 }
-            const float hpost = hq[a];
+            const float hpost = ONE ? q1 : qs[a];
 #pragma unroll
             for (int q = 0; q < V; ++q) {
                 const float py = hpost * y[q];
@@ -271,6 +289,8 @@ __global__ __launch_bounds__(256) void mhc_mix_kernel(MhcArgs m) {
             else
                 *op = v[0];
         }
+        c += blockDim.x * V;
+        if (c < dim) columns(c);
     }
 }
 
@@ -294,17 +314,37 @@ hipError_t launch_mhc_heads(const MhcArgs &m, int rows, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Output lanes a workgroup of the mix takes: one while those workgroups are few
+// (a row's lanes side by side, bound by a load's latency), all of them once
+// reading the stream again for each costs more, two between. Measured on MI355X
+// (us, one, two and all): 4 lanes of 512 at 1, 256, 512, 1000 and 12,000 rows
+// 2.5, 3.1, 3.9, 5.7, 100 against 2.7, 3.3, 3.7, 4.9, 56 and 3.2, 3.6, 4.2, 4.9,
+// 37; 8 of 512 at 37, 375 and 3000 3.0, 12.0, 80 against 3.3, 5.8, 44 and 6.0,
+// 7.1, 19; 4 of 64 at 512 and 3000 3.1, 6.2 against 3.2, 5.0 and 3.9, 4.7; 4 of
+// 2048 at 128 and 750 4.1, 26 against 4.5, 16 and 5.8, 13. All lanes at every
+// size, their coefficients read from memory, took 3.6 us for one row of 4 x 512.
+int mix_lanes(int lanes, int dim, int rows) {
+    const long long wgs = static_cast<long long>(rows) * lanes, values = wgs * dim;
+    if (wgs <= 1024 || (wgs <= 3072 && values <= 1 << 19)) return 1;
+    return lanes > 2 && values <= 3 << 19 ? 2 : lanes;
+}
+
 hipError_t launch_mhc_mix(const MhcArgs &m, int rows, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
     const uintptr_t all = reinterpret_cast<uintptr_t>(m.stream) | reinterpret_cast<uintptr_t>(m.out) |
                           reinterpret_cast<uintptr_t>(m.block_out) | reinterpret_cast<uintptr_t>(m.u);
     const int v = (m.dim & 3) == 0 && (all & 15) == 0 ? 4 : 1;  // float4s where every row is whole ones
     const int items = (m.dim + v - 1) / v, threads = items >= 256 ? 256 : (items + 63) / 64 * 64;
-    const dim3 grid(static_cast<unsigned>(rows)), block(threads);
-    if (v == 4)
-        hipLaunchKernelGGL((mhc_mix_kernel<4>), grid, block, 0, s, m);
+    const int per = mix_lanes(m.lanes, m.dim, rows);
+    const dim3 grid(static_cast<unsigned>(rows), static_cast<unsigned>((m.lanes + per - 1) / per)), block(threads);
+    if (v == 4 && per == 1)
+        hipLaunchKernelGGL((mhc_mix_kernel<4, true>), grid, block, 0, s, m, per);
+    else if (v == 4)
+        hipLaunchKernelGGL((mhc_mix_kernel<4, false>), grid, block, 0, s, m, per);
+    else if (per == 1)
+        hipLaunchKernelGGL((mhc_mix_kernel<1, true>), grid, block, 0, s, m, per);
     else
-        hipLaunchKernelGGL((mhc_mix_kernel<1>), grid, block, 0, s, m);
+        hipLaunchKernelGGL((mhc_mix_kernel<1, false>), grid, block, 0, s, m, per);
     return hipGetLastError();
 }
 

@@ -71,3 +71,18 @@ def test_heads_and_mix(lanes, dim, offset):
     ohp, ohq, ohr, ou = orc.mhc_heads(pre, post, res, stream, rows, lanes, dim, aff)
     for got, want in ((hp, ohp), (hq, ohq), (hr, ohr), (u, ou), (out, orc.mhc_mix(stream, ohr, ohq, block_out, ou, rows, lanes, dim))):
         assert same(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("lanes,dim,rows", [(4, 512, 256), (4, 512, 257), (4, 512, 769), (4, 64, 768), (4, 64, 769), (3, 70, 900),
+                                            (5, 128, 900), (8, 500, 150), (8, 5, 3000), (3, 1024, 600), (1, 512, 1100)])
+def test_mix_output_lanes(lanes, dim, rows):
+    # one, two and all output lanes a workgroup, a last one short of its two
+    import torch
+
+    g = np.random.default_rng(lanes + dim + rows)
+    f = lambda *s: g.standard_normal(s).astype(np.float32)
+    stream, hr, hq, block_out, u = f(rows, lanes, dim), f(rows, lanes, lanes), f(rows, lanes), f(rows, dim), f(rows, dim)
+    out = torch.full((rows, lanes, dim), 9.0, device="cuda")
+    needle.mhc_mix_dev(out, _t(stream), _t(hr), _t(hq), _t(block_out), _t(u), rows, lanes, dim)
+    torch.cuda.synchronize()
+    assert same(out.cpu().numpy(), orc.mhc_mix(stream, hr, hq, block_out, u, rows, lanes, dim))

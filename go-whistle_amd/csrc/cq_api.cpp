@@ -1004,15 +1004,34 @@ int run_few(cq_matrix *const *ms, int n, float *const *dsts, const float *x, int
     return CQ_OK;
 }
 
-// Workgroups (four 64-row blocks by four activations) from which Exact's
-// products take the four-activation kernel: below it its two barriers a group
-// leave the chip idle where a workgroup per activation spreads wider. Measured
-// on MI355X (us, one activation against four): 2048x512 CQ4 at 32, 64 and 128
-// activations (64, 128, 256 workgroups) 10.5, 15.7, 22.5 against 13.7, 13.9,
-// 14.6; 16384x512 CQ4 at 5 and 16 (128, 256) 12.5, 21.6 against 18.0, 14.5;
-// 512x2048 CQ2 at 128 and 375 (64, 188) 19.7, 71.3 against 31.5, 39.2; 96x512
-// CQ4 at 375 (94) 9.6 against 17.8.
-constexpr long long kExactQuadWgs = 160;
+// Whether Exact's products take the four-activation kernel, by its work in
+// whole workgroups: (64-row block, four activations) items over four, as a
+// workgroup's wavefronts past a matrix's blocks have none. Below the line its
+// two barriers a group leave the chip idle where a workgroup per activation
+// spreads wider; long inputs, whose tables that form builds in chunks, cross it
+// sooner; and the last rows % 4 activations, on lookupNibble's eight sums, set
+// a short launch's length (3 us at 4 groups), which the 2-bit tables, half as
+// many to build, make up for later. Measured on MI355X (us, a workgroup per
+// activation against four activations; items in brackets): 2048x512 CQ4 at 64,
+// 80, 95 and 128 activations (128, 160, 192, 256) 14.2, 17.1, 17.3, 20.4 against
+// 12.9, 13.0, 17.3, 13.2, in groups of 32 at 64 and 80 16.0, 19.5 against 16.9,
+// 17.1, CQ2 in groups of 64 at 80, 95 and 128 11.6, 11.6, 13.5 against 10.5,
+// 12.6, 10.5; 64x512 CQ4 at 1500 and 3000 (94, 188) 13.5, 23.8 against 16.3,
+// 21.7; 300x500 CQ4 at 320, 375 and 500 (100, 118, 156) 14.7, 14.8, 20.2 against
+// 12.8, 16.9, 13.1; 1001x1000 CQ4 at 64 and 96 (64, 96) 16.3, 32.9 against 23.6,
+// 23.9, CQ2 10.5, 15.9 against 16.2, 16.3; 512x2048 CQ4 at 128 and 192 (64, 96)
+// 48.4, 84.5 against 44.9, 45.6, CQ2 17.9, 35.4 against 30.2, 30.9.
+bool exact_quad_pays(cq_matrix *const *ms, int n, int rows) {
+    const CqStore &s = *ms[0]->st;
+    if (!exact_quad_geometry(s.group_bytes) || rows < 4) return false;
+    long long blocks = 0;
+    for (int k = 0; k < n; ++k)
+        blocks += (ms[k]->row0 + ms[k]->out + kBlockRows - 1) / kBlockRows - ms[k]->row0 / kBlockRows;
+    const long long work = blocks * ((rows + 3) / 4) / 4;
+    if (s.in >= (s.width == 4 ? 1000 : 1536)) return work >= 90;
+    if (rows % 4 == 0) return work >= (s.group_bytes == 64 ? 100 : 150);
+    return work >= (s.width == 2 && s.group < 256 && s.in < 1200 ? 224 : 150);
+}
 
 int run_product(cq_matrix *const *ms, int n, float *const *dsts, const float *x, int rows, hipStream_t stream,
                 const Fuse *fz = nullptr, const TabOut *to = nullptr, int *built = nullptr) {
@@ -1046,14 +1065,7 @@ int run_product(cq_matrix *const *ms, int n, float *const *dsts, const float *x,
     LaunchPlan p = plan(s0, mode, nblk_total, rows);
     if (p.lds > device_info().max_lds)
         return fail(CQ_ERR_UNSUPPORTED, "cq: a product of group %d needs %zu bytes of LDS", s0.group, p.lds);
-    bool quad = false;  // four activations a workgroup
-    if (mode == kModeExact && exact_quad_geometry(s0.group_bytes) && rows >= 4) {
-        long long wgs = 0;
-        for (int k = 0; k < n; ++k)
-            wgs += ((ms[k]->row0 + ms[k]->out + kBlockRows - 1) / kBlockRows - ms[k]->row0 / kBlockRows + 3) / 4;
-        wgs *= (rows + 3) / 4;
-        quad = wgs >= kExactQuadWgs;
-    }
+    const bool quad = mode == kModeExact && exact_quad_pays(ms, n, rows);  // four activations a workgroup
     a.tb = quad ? 4 : p.tb;
     a.gc = p.gc;
     int tiles = 0;

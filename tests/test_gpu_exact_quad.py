@@ -34,6 +34,17 @@ def test_exact_quads(bits, group, out, inp, rows):
     assert same(y.cpu().numpy(), o.gemm(x.reshape(-1), rows, orc.NIBBLE4))
 
 
+@pytest.mark.parametrize("bits,group,out,inp,rows", [
+    # either side of the work from which the four-activation kernel runs: 4 bits
+    # in whole fours and with a rest, 2 bits with a rest, long inputs, blocks
+    # that leave wavefronts of a tile idle
+    (4, 128, 512, 500, 199), (4, 128, 512, 500, 200), (4, 128, 512, 500, 297), (4, 128, 512, 500, 298),
+    (2, 64, 512, 300, 300), (2, 64, 512, 300, 301), (2, 64, 512, 300, 445), (2, 64, 512, 300, 446),
+    (4, 32, 70, 1000, 716), (4, 32, 70, 1000, 720), (2, 256, 300, 1600, 284), (2, 256, 300, 1600, 288)])
+def test_exact_either_side_of_the_line(bits, group, out, inp, rows):
+    test_exact_quads(bits, group, out, inp, rows)
+
+
 def test_views_and_special_values():
     import torch
 

@@ -1883,6 +1883,49 @@ size_t chain_lds(const AttendArgs &a, int jc, int rs) {
 // The resident form also holds the two product buffers behind the rows.
 size_t chain_res_lds(const AttendArgs &a, int rs) { return chain_lds(a, 64, rs) + 2 * sizeof(float) * kProdFloats; }
 
+// Wavefronts (pairs) of a workgroup of the prompt form for prompts of more
+// (row, head) pairs than stay resident, or 0 where the other forms are the
+// better ones; lds and wgs get its LDS (with_pages as launch_attend_int8's) and
+// workgroups. A workgroup takes 4 to 16 pairs, about one workgroup for each CU.
+// The prompt form pays the staging of every key once a workgroup, the others a
+// wavefront's own reads a pair, so it loses
+//  - over few keys, unless there are pairs enough (64-code key heads go to the
+//    ring, the others to the slower chain kernel): over 2 key heads of 64, 64
+//    streams x 2 rows over 32 and 64 keys 7.2, 7.7 us against the ring's 5.9, 6.8,
+//    256 x 4 rows over 48 14.9 against 17.3; of 48 codes 7.2, 7.7 against 6.1, 6.7
+//    and 14.2 against 21.5;
+//  - where more workgroups than CUs leave fewer than 16 of its wavefronts on a
+//    CU, or stage for four pairs each: 128 streams x 4 rows over 8 key heads of
+//    64, 128, 160 and 448 keys 12.3, 19.0, 62 us against the ring's 13.1, 15.4, 33;
+//    256 x 4 rows over 2 key heads of 64, 560 keys (14 pairs a workgroup, LDS for
+//    one on a CU) 84 against 60, but 16 streams x 32 rows, which share more keys,
+//    33 against 39; key heads of 48, 128 x 4 rows over 8, 448 keys (two workgroups
+//    of four pairs do not fit a CU) 57 against 36, 160 keys 13.7 against 19.5.
+// (MI355X, us a call from a graph, 8 heads, causal spans.)
+template <class Pages>
+int rows_waves(const AttendArgs &a, int cus, Pages with_pages, size_t &lds, long long &wgs) {
+    constexpr size_t most = 150 * 1024;
+    const int kv_heads = a.k_cols / a.qk, pairs = a.t * (a.heads / kv_heads);
+    const long long groups = static_cast<long long>(a.batch) * kv_heads, total = groups * pairs;
+    int nw = static_cast<int>(std::min<long long>(kRowsMaxWaves, std::max(4LL, (total + cus - 1) / cus)));
+    nw = std::min(nw, pairs);
+    while (nw > 4 && with_pages(rows_lds(a, nw)) > most) --nw;
+    lds = with_pages(rows_lds(a, nw));
+    if (nw < 4 || lds > most) return 0;
+    wgs = groups * ((pairs + nw - 1) / nw);
+    if (wgs > grid_limit(64 * nw)) return 0;
+    const bool ring = a.qk == kChainVd, many = wgs > cus;
+    const int on_cu = static_cast<int>(most / lds);
+    bool pays = true;
+    if (a.nk_max <= (ring ? 80 : 64))
+        pays = ring ? total > 24LL * cus : many || nw >= 12;
+    else if (many && ring)
+        pays = nw >= 8 ? a.t >= 16 || nw * on_cu >= 16 : on_cu >= 5;
+    else if (many)
+        pays = nw >= 8 || on_cu >= 2;
+    return pays ? nw : 0;
+}
+
 hipError_t launch_attend_int8(const AttendArgs &args, int cus, hipStream_t stream) {
     AttendArgs a = args;
     if (a.t <= 0 || a.heads <= 0 || a.batch <= 0) return hipSuccess;
@@ -1905,24 +1948,16 @@ hipError_t launch_attend_int8(const AttendArgs &args, int cus, hipStream_t strea
             const size_t lds = with_pages(chain_res_lds(a, rs));
             if (lds <= 150 * 1024) return launch_attend_chain<4, 64, true>(a, rs, lds, stream);
         }
-        // Prompts of more workgroups than stay resident: a workgroup of 4 to 16
-        // pairs, about one for each CU. Fewer than eight wavefronts need a CU
-        // each, or LDS for two workgroups on one: 128 streams x 4 rows of 8
-        // key heads took 65 us with four alone on a CU, 39 the way below.
         if (a.t > 1) {
-            const int kv_heads = a.k_cols / a.qk, pairs = a.t * (a.heads / kv_heads);
-            const long long groups = static_cast<long long>(a.batch) * kv_heads, total = groups * pairs;
-            int nw = static_cast<int>(std::min<long long>(kRowsMaxWaves, std::max(4LL, (total + cus - 1) / cus)));
-            nw = std::min(nw, pairs);
-            while (nw > 4 && with_pages(rows_lds(a, nw)) > 150 * 1024) --nw;
-            const int per_group = (pairs + nw - 1) / nw;
-            const size_t lds = with_pages(rows_lds(a, nw));
-            const bool enough = nw >= 8 || groups * per_group <= cus || 2 * lds <= 150 * 1024;
-            if (nw >= 4 && enough && lds <= 150 * 1024 && groups * per_group <= grid_limit(64 * nw)) {
+            size_t lds = 0;
+            long long wgs = 0;
+            const int nw = rows_waves(a, cus, with_pages, lds, wgs);
+            if (nw > 0) {
                 static std::atomic<unsigned long long> attr{0};
                 if (hipError_t e = lds_limit_once(reinterpret_cast<const void *>(&attend_rows_kernel), 152 * 1024, attr)) return e;
-                hipLaunchKernelGGL(attend_rows_kernel, dim3(static_cast<unsigned>(groups * per_group)), dim3(64 * nw), lds, stream,
-                                   a, per_group);
+                const int pairs = a.t * (a.heads / (a.k_cols / a.qk));
+                hipLaunchKernelGGL(attend_rows_kernel, dim3(static_cast<unsigned>(wgs)), dim3(64 * nw), lds, stream, a,
+                                   (pairs + nw - 1) / nw);
                 return hipGetLastError();
             }
         }

@@ -4,8 +4,8 @@ Bit for bit against the oracle at the edges of what the kernel splits by:
 the pairs of a workgroup (4 to 16, with a last one that is not full), the
 32-key blocks and the four keys of a weight read, two spans in any order and
 at any distance, empty spans and spans off the cache, RoPE of the query,
-shared and paged caches, infinite scales; key counts past its LDS go to the
-other kernels."""
+shared and paged caches, infinite scales; few keys, and key counts past its
+LDS, go to the other kernels."""
 
 import numpy as np
 import pytest
@@ -54,6 +54,14 @@ def _spans(kind, g, batch, t, nk):
     (130, 4, 8, 8, 64, 448, True, "causal", "plain"),   # four pairs a workgroup, too many of them
     (2, 80, 8, 2, 64, 900, True, "causal", "plain"),    # past the LDS
     (3, 40, 8, 2, 64, 70, True, "two", "inf"),
+    # few keys and pairs enough for the kernel, and either side of the fewest keys
+    # it takes below that
+    (128, 4, 8, 1, 48, 3, True, "two", "plain"),
+    (256, 4, 8, 8, 64, 20, True, "two", "plain"),
+    (5, 27, 4, 1, 16, 65, True, "two", "rope"),
+    (5, 27, 4, 1, 16, 64, True, "two", "rope"),
+    (7, 19, 4, 4, 32, 70, True, "two", "shared"),
+    (3, 40, 8, 2, 64, 81, True, "two", "inf"),
 ])
 def test_prompt_rows_bit_exact(batch, t, heads, kv_heads, qk, nk, quant, kind, form):
     import torch

@@ -1,8 +1,8 @@
 """Int8 attention of prompts (t > 1, more (row, head) pairs than stay
 resident): several pairs a workgroup over keys and values staged once.
 Bit for bit against the oracle at the edges of what the kernel splits by:
-the pairs of a workgroup (4 to 16, with a last one that is not full), the
-32-key blocks and the four keys of a weight read, two spans in any order and
+the pairs of a workgroup (4 to 16, with a last one that is not full, and fewer
+where the LDS ends), the 32-key blocks and the four keys of a weight read, two spans in any order and
 at any distance, empty spans and spans off the cache, RoPE of the query,
 shared and paged caches, infinite scales; few keys, and key counts past its
 LDS, go to the other kernels."""
@@ -54,6 +54,12 @@ def _spans(kind, g, batch, t, nk):
     (130, 4, 8, 8, 64, 448, True, "causal", "plain"),   # four pairs a workgroup, too many of them
     (2, 80, 8, 2, 64, 900, True, "causal", "plain"),    # past the LDS
     (3, 40, 8, 2, 64, 70, True, "two", "inf"),
+    # 16 wavefronts a workgroup, whole and with a last one of 4; cut to 14 by the
+    # LDS, without and with a page table in it
+    (4, 128, 8, 2, 48, 448, True, "two", "plain"),
+    (13, 85, 4, 1, 64, 200, True, "two", "plain"),
+    (16, 32, 8, 2, 64, 560, True, "two", "plain"),
+    (16, 33, 8, 2, 64, 560, False, "two", "paged"),
     # few keys and pairs enough for the kernel, and either side of the fewest keys
     # it takes below that
     (128, 4, 8, 1, 48, 3, True, "two", "plain"),

@@ -366,7 +366,8 @@ int nd_add_dev(float *x, const float *y, long long n, void *stream);
  * {w1a, w1b, w2a, w2b, w3a, w3b} row-major, cond_v dim x rank, cond_u
  * rank x n, p1 and p2 permutations of n (hada_p1/p2). n <= 1024, rank <= 32.
  * Float32, within 1e-5 of the float64 form (hadamard_test.go:152-191); the
- * reference's GEMMs sum in their library's own order. */
+ * reference's GEMMs sum in their library's own order. The order here follows
+ * na and nb alone: a row's result is the same in every call. */
 int nd_hadamard_mlp_dev(float *out, const float *x, int rows, int dim, int na, int nb, int rank,
                         const float *const *vecs, const float *const *factors, const float *cond_v,
                         const float *cond_u, const int32_t *p1, const int32_t *p2, void *stream);

@@ -50,3 +50,24 @@ def test_nan_and_inf_stay_in_their_rows():
         want = hr.forward(w, x[r:r + 1], 1)[0]
         assert np.max(np.abs(y[r] - want)) <= 1e-5 * max(1.0, np.max(np.abs(want)))
     assert np.isnan(y[1]).all() and not np.isfinite(y[2]).any()
+
+
+@pytest.mark.parametrize("na,nb,rank,dim", [(16, 16, 8, 256), (16, 32, 8, 511), (32, 16, 5, 512), (32, 32, 16, 1024),
+                                            (24, 32, 16, 768), (17, 3, 1, 40), (40, 5, 3, 200)])
+def test_rows_do_not_depend_on_the_call(na, nb, rank, dim):
+    # a row's bits are the same alone, in a long call and off a 16-byte line,
+    # and with weights off it
+    import torch
+
+    g = np.random.default_rng(na + nb + rank + dim)
+    w = hr.random_weights(g, na, nb, rank, dim)
+    m = needle.HadamardMLP(w)
+    rows, few = 2100, 6
+    x = torch.from_numpy(g.standard_normal((rows, dim)).astype(np.float32)).cuda()
+    z = lambda n: torch.zeros(n + 4, device="cuda")[1:n + 1]
+    many, some, off = torch.zeros(rows, dim, device="cuda"), torch.zeros(few, dim, device="cuda"), z(few * dim)
+    m.forward_dev(many, x, rows)
+    m.forward_dev(some, x, few)
+    m.forward_dev(off, z(few * dim).copy_(x[:few].reshape(-1)), few)
+    bits = lambda t: t.reshape(-1)[:few * dim].view(torch.int32)
+    assert torch.equal(bits(many), bits(some)) and torch.equal(bits(some), bits(off))

@@ -368,7 +368,6 @@ __global__ __launch_bounds__(256) void hadamard_wave_kernel(HadaArgs h, int rows
         for (int ta = 0; ta < TA; ++ta)
 #pragma unroll
             for (int s = 0; s < S; ++s) cond[ta][s] = 0.0f;
-#pragma unroll 4
         for (int r = 0; r < rank; ++r) {
             const float p = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, prob), r));
 #pragma unroll

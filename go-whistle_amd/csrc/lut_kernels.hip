@@ -482,27 +482,17 @@ __device__ __forceinline__ void next_tables(const TabOut &o, const float *yo, un
     CQ_GLOBAL int8_t *tab = gptr_w(o.tab) + (static_cast<size_t>(t >> 5) * groups) * NP * 2048 + (t & 31) * 16;
     for (int it = tid; it < groups * NJ; it += 64 * W) {
         const int g = it / NJ, j = it - g * NJ;
-        float x0, x1 = 0.0f;
-        if constexpr (TB == 4) {
-            x0 = av[g * AP + j];
-        } else {
-            x0 = av[g * AP + 2 * j];
-            x1 = av[g * AP + 2 * j + 1];
-        }
+        const float x0 = av[g * AP + 2 * j], x1 = av[g * AP + 2 * j + 1];
         uint32_t lo[4], hi[4];
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
             uint32_t b[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
+            for (int q = 0; q < 4; ++q) {  // code = hi << 2 | lo
                 const int code = 4 * qd + q;
-                if constexpr (TB == 4) {
-                    b[q] = rne_bits(cbv[code] * x0);
-                } else {  // code = hi << 2 | lo
-                    const float l = cbv[code & 3] * x0, h = cbv[code >> 2] * x1;
-                    const float sm = l + h;
-                    b[q] = rne_bits(sm);
-                }
+                const float l = cbv[code & 3] * x0, h = cbv[code >> 2] * x1;
+                const float sm = l + h;
+                b[q] = rne_bits(sm);
             }
             planes4(b[0], b[1], b[2], b[3], lo[qd], hi[qd]);
         }

@@ -1340,27 +1340,17 @@ __global__ __launch_bounds__(256) void lut_tables_kernel(TabArgs a) {
 #pragma unroll
     for (int k = 0; k < NJ / PS; ++k) {
         const int j = jb + PS * k;
-        float x0, x1 = 0.0f;
-        if constexpr (BITS == 4) {
-            x0 = av[tt * AP + j];
-        } else {
-            x0 = av[tt * AP + 2 * j];
-            x1 = av[tt * AP + 2 * j + 1];
-        }
+        const float x0 = av[tt * AP + 2 * j], x1 = av[tt * AP + 2 * j + 1];
         uint32_t lo[4], hi[4];
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
             uint32_t b[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
+            for (int q = 0; q < 4; ++q) {  // code = hi << 2 | lo
                 const int code = 4 * qd + q;
-                if constexpr (BITS == 4) {
-                    b[q] = rne_bits(cbv[code] * x0);
-                } else {  // code = hi << 2 | lo
-                    const float l = cbv[code & 3] * x0, h = cbv[code >> 2] * x1;
-                    const float sm = l + h;
-                    b[q] = rne_bits(sm);
-                }
+                const float l = cbv[code & 3] * x0, h = cbv[code >> 2] * x1;
+                const float sm = l + h;
+                b[q] = rne_bits(sm);
             }
             planes4(b[0], b[1], b[2], b[3], lo[qd], hi[qd]);
         }
@@ -1660,7 +1650,7 @@ __device__ __forceinline__ void sa_wait_vm(int n) {
 template <int BITS>
 constexpr size_t sa_lds_bytes() {
     return static_cast<size_t>(kSaSlots) * kSaSlot + kSaBlocks * MfmaGeo<BITS>::UPG * 1024 + kSaBlocks * 128 +
-           kSaBlocks * 128 + 256;
+           kSaBlocks * 128 + (BITS == 2 ? 256 : 0);  // 2 bits: the one-hot table
 }
 
 template <int BITS>
@@ -1925,7 +1915,7 @@ __global__ __launch_bounds__(64 * kSaBlocks, 2) void lut_mfma_tabs_kernel(LutLau
 
 template <int BITS>
 size_t tab_lds_bytes(int groups) {
-    return sizeof(float) * static_cast<size_t>(groups) * 32 * 64 + 16 * 16;
+    return sizeof(float) * static_cast<size_t>(groups) * 32 * 64 + (BITS == 2 ? 16 * 16 : 0);  // 2 bits: the one-hot table
 }
 
 template <int BITS>

@@ -728,39 +728,34 @@ int run_split(cq_matrix *const *ms, int n, float *const *dsts, const float *x, i
 // 64-row block stream them. A workgroup reads its 32 activations' tables
 // whole (8 KiB per activation and 512 inputs), so the form pays where the
 // lut kernel's work, linear in rows x activations, outgrows the form's
-// ~15 us floor at these sizes (from about 256K row-activations at 4 bits,
+// ~10 us floor at these sizes (from about 256K row-activations at 4 bits,
 // 384K at 2, and 16 activations), or where its (block, tile) workgroups
 // reach the CUs; past 3072 activations over 768 rows or more, at 2 bits,
-// or up to 6144 activations (a 512-row CQ4 matrix's tables, read by few
-// blocks, cost more than the 512-row MFMA form's own table builds at 12000).
-// Measured on MI355X when the lines were drawn (pre-pass + product against
-// the form chosen otherwise; the 4-bit split into planes and residuals has
-// since made the form's times 0.5-0.75 of these, see lut_mfma_tab_kernel): at 256 activations the four 512x512 CQ4 q/k/v/gate products
-// with the norm 18.6 against 28.2 us, 2048x512 CQ2 with the norm and SiLU
-// 16.0 against 19.1 us, the 16384x512 head 60.2 against 64.4 us, 1536x512
-// CQ4 16.2 against 23.5 us, 1024x512 CQ4 15.9 against 16.7 us, but 1024x512
-// CQ2 12.0 against 10.8 us and a 512x512 CQ4 product 14.9 against 9.6 us;
-// the 16384x512 CQ4 head at 16, 32, 64 and 95 activations 15.5, 15.7, 22.6,
-// 30.3 us against 16.8, 28.0, 50.4, 70.1 us (CQ2 at 32 and 64 12.1 and 16.0
-// against 17.7 and 30.4 us);
-// 2048x512 CQ4 at 64, 96, 192 activations 14.7, 16.1, 17.5 us against the
-// lut kernel's 10.8, 17.0, 26.8 us; at 375, 1024, 1500, 3000, 6000 and
-// 12000 activations 25.8, 44.0, 57.5, 107.1, 194.4, 361.1 us against 31.4,
-// 57.7, 67.5, 118.0, 244.0, 363.8 us (split, split, then the 512-row MFMA
-// form), CQ2 at 375, 1500, 6000, 12000 16.9, 36.7, 106.7, 203.4 against
-// 25.5, 43.9, 154.3, 236.1 us; 1024x512 CQ4 at 1500, 6000, 12000 37.5,
-// 101.7, 202.2 us against 43.2, 114.4, 220.3 us; 512x512 CQ4 at 12000 120.3
-// against the MFMA form's 111.4 us, but at 4000 and 6000 activations 50.9
-// and 68.5 us against the split form's 53.8 and 75.3 us (CQ2 at 4000, 6000,
-// 12000: 35.8, 45.6, 73.9 against 52.8, 74.8, 83.8 us); 768x512 CQ4 at 4000,
-// 6000, 12000 62.2, 85.7, 162.6 us against the MFMA form's 70.2, 117.9,
-// 225.6 us; small matrices past 3072 activations keep the form at 2 bits
-// (64x512 CQ2 at 3500 / 12000: 23.5 / 40.8 against the MFMA form's 40.5 /
-// 77.3 us, 384x512 CQ2 at 12000 70.1 against 79.0 us) and at 4 bits to
-// 6144 (64x512 CQ4 at 6000: 40.2 against 62.4 us; at 12000 the two are
-// within 1%). The views must share their tables (one
-// pre-pass serves them all). The tables live in a leased workspace (at 12288
-// activations of 1024 inputs, 384 MiB).
+// or up to 6144 activations. The 4-bit lines date from tables of both int8
+// planes, twice the bytes and twice the MFMAs, so they lie on the safe side
+// of today's (marked *: the form would win there and is not taken).
+// Measured on MI355X (us, pre-pass + product against the form chosen
+// otherwise, graph-replayed): the 16384x512 CQ4 head at 16, 32, 64, 95 and
+// 256 activations 10.9, 11.2, 15.1, 19.6, 36.7 against 16.8, 26.4, 45.0,
+// 70.2, 67.3, CQ2 10.5, 10.9, 14.6, 18.9, 34.3 against 10.4, 15.1, 24.8,
+// 31.8, 43.3; 2048x512 CQ4 at 64, 96*, 128, 192 and 375 10.1, 10.4, 10.5,
+// 11.2, 15.1 against 9.8, 15.9, 15.3, 23.4, 28.5, at 1024, 1500, 3000, 6000
+// and 12000 26.3, 35.2, 53.6, 95.2, 177 against 51.7, 63.1, 112, 220, 336,
+// CQ2 at 128, 192, 375, 1500, 6000 and 12000 10.3, 11.0, 14.9, 34.7, 90.4,
+// 169 against 10.5, 16.1, 21.8, 43.5, 152, 233; 1536x512 CQ4 at 128* and 192
+// 10.3, 10.7 against 13.3, 17.5; 1024x512 CQ4 at 128, 192*, 256 and 12000
+// 10.3, 10.7, 10.7, 109 against 9.8, 15.4, 15.2, 219, CQ2 at 256, 375*, 512
+// and 4000 10.5, 11.4, 11.9, 45.9 against 10.6, 13.5, 15.5, 44.0; 768x512
+// CQ4 at 192*, 256*, 375 and 12000 10.6, 10.5, 11.6, 95.5 against 11.7, 13.5,
+// 18.8, 219; 512x512 CQ4 at 256, 375*, 512, 6000 and 12000* 10.5, 11.5, 11.9,
+// 45.3, 74.9 against 10.0, 17.9, 18.7, 66.0, 113, CQ2 at 512, 1500, 3000 and
+// 12000 11.5, 20.5, 30.3, 64.8 against 10.8, 20.0, 35.6, 76.9; 64x512 CQ4 at
+// 3500, 6000 and 12000* 25.8, 31.3, 50.3 against 24.1, 33.8, 108, CQ2 24.2,
+// 27.8, 40.5 against 15.4, 23.7, 72.1. With the norm in front: the four
+// 512x512 CQ4 q/k/v/gate products at 256 13.0 against 26.0, 2048x512 CQ2 with
+// SiLU 14.6 against 19.1. The views must share their tables (one pre-pass
+// serves them all). The tables live in a leased workspace (at 12288
+// activations of 1024 inputs, 192 MiB).
 constexpr int kTabMinRows = 16;
 constexpr int kTabMaxRows = 3072;       // any row count
 constexpr int kTabMaxRowsWide = 12288;  // over kTabWideBlocks blocks, at 2 bits, or to kTabMidRows

@@ -1528,14 +1528,13 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
 //
 // Bound by VALU issue (1,667 instructions a pair of 448 keys, busy 61% of the
 // kernel) behind one exposed staging. Measured on MI355X, 8 heads of 64, 448
-// keys a stream, causal, against a wavefront a pair reading its own rows (the
-// chain kernel at 48 codes a key head, the ring at 64): 4 streams x 96 rows, 2
-// key heads of 48 codes 31.3 -> 20.8 us (int8 values, converted by each pair,
-// 21.9); 8 key heads of 64 22.4 -> 18.5; 16 streams x 32 rows 36.2 -> 23.2 (8
-// key heads of 64 35.1 -> 24.0); 64 streams x 2 rows 20.5 -> 18.0; the closest,
-// 64 streams x 8 rows of 8 key heads of 64, 35.3 against 35.9. Loading a thread's
-// whole share before its first store, the query's with it: 21.5 (92 registers
-// for 60).
+// keys a stream, causal spans past the prompts' offsets, us a call from a graph
+// against the chain kernel (48 codes a key head) and the ring (64): 4 streams x
+// 96 rows over 2 key heads of 48 codes 29.5 -> 18.6, over 8 of 64 24.2 -> 19.6; 16
+// streams x 32 rows 37.3 -> 20.2, 8 key heads of 64 37.8 -> 21.7; rows_waves has
+// the calls where those are the better ones. int8 values, converted by each
+// pair, and a thread's whole share loaded before its first store, the query's
+// with it (92 registers for 60), were 5% and 3% slower.
 constexpr int kRowsMaxWaves = 16;
 
 using half2v = __attribute__((ext_vector_type(2))) _Float16;

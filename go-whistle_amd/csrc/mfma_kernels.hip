@@ -1370,8 +1370,9 @@ __global__ __launch_bounds__(256) void lut_tables_kernel(TabArgs a) {
 // split): 2048x512 CQ4 at 12,000 activations 309 -> 178 us, at 1,500 53.4 ->
 // 36 us, at 256 16.4 -> 12.4 us; the 16384x512 head at 256 64.5 -> 35 us; the
 // batch-256 decode step 1.525 -> 1.443 ms. What bounds the large ones now is
-// issue: the MFMAs are busy 48% of the cycles, VALU takes as many (the
-// one-hots' shifts and masks, the fold's 5 operations a sum).
+// issue: at 12,000 activations the MFMAs are busy 42% of the product's cycles,
+// and the VALU shares the SIMDs (the one-hots' shifts and masks, the fold's 5
+// operations a sum); a wavefront waits 37% of its time.
 //
 // The product: a workgroup per (64-row block, 32-activation tile), a
 // tile's workgroups on one XCD (or two), which shares their tables in its L2.

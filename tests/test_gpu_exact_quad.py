@@ -20,7 +20,8 @@ def same(a, b):
 
 
 @pytest.mark.parametrize("bits,group", [(4, 16), (4, 32), (4, 64), (4, 128), (4, 256), (2, 32), (2, 64), (2, 128), (2, 256)])
-@pytest.mark.parametrize("out,inp,rows", [(700, 300, 212), (700, 300, 213), (64, 130, 643), (1050, 256, 130)])
+@pytest.mark.parametrize("out,inp,rows", [(700, 300, 212), (700, 300, 213), (64, 130, 643), (1050, 256, 130),  # some below its line
+                                          (700, 300, 300), (700, 300, 333), (64, 130, 2400), (64, 130, 3603), (1050, 256, 210)])
 def test_exact_quads(bits, group, out, inp, rows):
     import torch
 

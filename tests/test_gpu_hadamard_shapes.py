@@ -1,8 +1,9 @@
-"""HadamardMLP on a wavefront per row (hadamard_wave_kernel) over the shapes
-it branches on: one and two tiles of 16 per factor, factors that fill them and
-not, widths cut inside a float4, ranks that are no multiple of 8, rows off a
-16-byte line, and factors and row counts it leaves to the workgroup form; within 1e-5 of the
-float64 form (internal/needle/hadamard_test.go:152-191)."""
+"""HadamardMLP's two forms over the shapes they branch on: factors of 16 and 32
+(a wavefront a row, one and two tiles of 16 a factor) and others (a workgroup a
+row), widths cut inside a float4, ranks that are no multiple of 8, rows off a
+16-byte line, few rows and many; within 1e-5 of the float64 form
+(internal/needle/hadamard_test.go:152-191). A row's bits are the same in every
+call."""
 
 import numpy as np
 import pytest

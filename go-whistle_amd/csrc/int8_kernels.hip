@@ -211,8 +211,8 @@ __global__ __launch_bounds__(kAttThreads) void attend_kernel(AttendArgs a) {
     const int lo0 = sp[0], len0 = sp[1] - sp[0], lo1 = sp[2], len1 = sp[3] - sp[2];
     const int n = len0 + len1;
     const long long kb = attend_cache_of(a, b);  // the cache this stream reads
-    if (kb < 0 || lo0 < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
-        return;  // spans off the cache, or no cache
+    if (kb < 0 || (lo0 | (a.nk_max - n)) < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
+        return;  // spans off the cache or overlapping past the logits' nk_max places, or no cache
     attend_stage_pages(a, b, smem);  // paged: the stream's page table into LDS
     const int32_t *pgs = reinterpret_cast<const int32_t *>(smem + a.page_lds);
 
@@ -531,8 +531,8 @@ __global__ __launch_bounds__(kAttThreads) void attend_stream_kernel(AttendArgs a
     const int lo0 = sp[0], len0 = sp[1] - sp[0], lo1 = sp[2], len1 = sp[3] - sp[2];
     const int n = len0 + len1;
     const long long kb = attend_cache_of(a, b);  // the cache this stream reads
-    if (kb < 0 || lo0 < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
-        return;  // spans off the cache, or no cache
+    if (kb < 0 || (lo0 | (a.nk_max - n)) < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
+        return;  // spans off the cache or overlapping past the logits' nk_max places, or no cache
     float *outp = a.out + b * a.out_stride + (static_cast<long long>(i) * a.heads + h) * VD;
     if (n == 0) {
         if (tid < VD) outp[tid] = 0.0f;
@@ -883,8 +883,8 @@ __global__ __launch_bounds__(64 * NW) void attend_chain_kernel(AttendArgs a, int
     const int lo0 = sp[0], len0 = sp[1] - sp[0], lo1 = sp[2], len1 = sp[3] - sp[2];
     const int n = len0 + len1;
     const long long kb = attend_cache_of(a, b);  // the cache this stream reads
-    if (kb < 0 || lo0 < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
-        return;  // spans off the cache, or no cache
+    if (kb < 0 || (lo0 | (a.nk_max - n)) < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
+        return;  // spans off the cache or overlapping past the logits' nk_max places, or no cache
     float *outp = a.out + b * a.out_stride + (static_cast<long long>(i) * a.heads + h) * kChainVd;
     if (n == 0) {
         if (tid < kChainVd) outp[tid] = 0.0f;
@@ -1284,8 +1284,8 @@ __global__ __launch_bounds__(64) void attend_ring_kernel(AttendArgs a, int swz) 
     const int lo0 = sp[0], len0 = sp[1] - sp[0], lo1 = sp[2], len1 = sp[3] - sp[2];
     const int n = len0 + len1;
     const long long kb = attend_cache_of(a, b);  // the cache this stream reads
-    if (kb < 0 || lo0 < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
-        return;  // spans off the cache, or no cache
+    if (kb < 0 || (lo0 | (a.nk_max - n)) < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
+        return;  // spans off the cache or overlapping past the logits' nk_max places, or no cache
     float *outp = a.out + b * a.out_stride + (static_cast<long long>(i) * a.heads + h) * ROW;
     if (n == 0) {
         outp[lane] = 0.0f;

@@ -269,8 +269,8 @@ int kv_reorder_noalloc_dev(int8_t *q, float *s, const int32_t *parent, const int
  * two ascending disjoint key spans {lo0, hi0, lo1, hi1}), and writes t rows
  * of heads*vd floats at out + b*out_stride (out_stride and q_stride 0 mean
  * dense streams; kv_stride and s_stride 0 share one cache). nk_max is the
- * number of key rows each stream's arrays hold: spans outside [0, nk_max)
- * leave that output untouched. quant_q chooses the int8 query
+ * number of key rows each stream's arrays hold: spans outside [0, nk_max),
+ * or of more than nk_max keys together, leave that output untouched. quant_q chooses the int8 query
  * (int8Logits, int8.go:278-285) or the float32 query (dotsF32I8,
  * int8.go:289-300). The softmax is softmaxInPlace (load.go:128-138) with
  * the amd64 kernel's exponent (exp_amd64.s:68-124). */

@@ -211,7 +211,7 @@ __global__ __launch_bounds__(kAttThreads) void attend_kernel(AttendArgs a) {
     const int lo0 = sp[0], len0 = sp[1] - sp[0], lo1 = sp[2], len1 = sp[3] - sp[2];
     const int n = len0 + len1;
     const long long kb = attend_cache_of(a, b);  // the cache this stream reads
-    if (kb < 0 || (lo0 | (a.nk_max - n)) < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
+    if (kb < 0 || lo0 < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max || n > a.nk_max)
         return;  // spans off the cache or overlapping past the logits' nk_max places, or no cache
     attend_stage_pages(a, b, smem);  // paged: the stream's page table into LDS
     const int32_t *pgs = reinterpret_cast<const int32_t *>(smem + a.page_lds);
@@ -531,7 +531,7 @@ __global__ __launch_bounds__(kAttThreads) void attend_stream_kernel(AttendArgs a
     const int lo0 = sp[0], len0 = sp[1] - sp[0], lo1 = sp[2], len1 = sp[3] - sp[2];
     const int n = len0 + len1;
     const long long kb = attend_cache_of(a, b);  // the cache this stream reads
-    if (kb < 0 || (lo0 | (a.nk_max - n)) < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
+    if (kb < 0 || lo0 < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max || n > a.nk_max)
         return;  // spans off the cache or overlapping past the logits' nk_max places, or no cache
     float *outp = a.out + b * a.out_stride + (static_cast<long long>(i) * a.heads + h) * VD;
     if (n == 0) {
@@ -883,7 +883,7 @@ __global__ __launch_bounds__(64 * NW) void attend_chain_kernel(AttendArgs a, int
     const int lo0 = sp[0], len0 = sp[1] - sp[0], lo1 = sp[2], len1 = sp[3] - sp[2];
     const int n = len0 + len1;
     const long long kb = attend_cache_of(a, b);  // the cache this stream reads
-    if (kb < 0 || (lo0 | (a.nk_max - n)) < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max)
+    if (kb < 0 || lo0 < 0 || len0 < 0 || sp[1] > a.nk_max || lo1 < 0 || len1 < 0 || sp[3] > a.nk_max || n > a.nk_max)
         return;  // spans off the cache or overlapping past the logits' nk_max places, or no cache
     float *outp = a.out + b * a.out_stride + (static_cast<long long>(i) * a.heads + h) * kChainVd;
     if (n == 0) {
@@ -1897,8 +1897,10 @@ size_t chain_res_lds(const AttendArgs &a, int rs) { return chain_lds(a, 64, rs) 
 //    CU, or stage for four pairs each: 128 streams x 4 rows over 8 key heads of
 //    64, 128, 160 and 448 keys 12.3, 19.0, 62 us against the ring's 13.1, 15.4, 33;
 //    256 x 4 rows over 2 key heads of 64, 560 keys (14 pairs a workgroup, LDS for
-//    one on a CU) 84 against 60, but 16 streams x 32 rows, which share more keys,
-//    33 against 39; key heads of 48, 128 x 4 rows over 8, 448 keys (two workgroups
+//    one on a CU) 84 against 60; prompts of 8 rows and more, whose pairs share
+//    more keys, keep it: 16 streams x 32 rows 33 against 39, 64 x 8 rows over 8 key
+//    heads, 480 keys 35 against 33, 550 keys that every row sees 45 against 56; key
+//    heads of 48, 128 x 4 rows over 8, 448 keys (two workgroups
 //    of four pairs do not fit a CU) 57 against 36, 160 keys 13.7 against 19.5.
 // (MI355X, us a call from a graph, 8 heads, causal spans.)
 template <class Pages>
@@ -1919,7 +1921,7 @@ int rows_waves(const AttendArgs &a, int cus, Pages with_pages, size_t &lds, long
     if (a.nk_max <= (ring ? 80 : 64))
         pays = ring ? total > 24LL * cus : many || nw >= 12;
     else if (many && ring)
-        pays = nw >= 8 ? a.t >= 16 || nw * on_cu >= 16 : on_cu >= 5;
+        pays = nw >= 8 ? a.t >= 8 || nw * on_cu >= 16 : on_cu >= 5;
     else if (many)
         pays = nw >= 8 || on_cu >= 2;
     return pays ? nw : 0;
